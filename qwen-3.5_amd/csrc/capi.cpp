@@ -79,6 +79,49 @@ size_t acc_bytes(const q35_dims& d, int B) {
   return std::max(gdn, std::max(att, mlp));
 }
 
+// ---- the multi-row path of the layer calls and q8_gemv (mvm.hip), unless a buffer's alignment or
+// a shape asks for the one-row kernel's row groups.  Layer calls take it from 2 rows on (device time
+// of the 2B MLP at 2 rows 27.9 -> 24.0 us from KN weights, 27.3 -> 20.8 tiled; attention 30.0 -> 25.9,
+// DeltaNet 28.2 -> 21.7); q8_gemv from 4 rows, where the one launch of the one-row kernel takes as
+// long as the two launches' host time (2048 x 6144 at 4 rows: 14.0 -> 9.4 us on the device, 14.45
+// issued one by one either way; at 2 rows 12.9 against 14.7 issued one by one).
+constexpr int kMvmMin = 2, kMvmGemvMin = 4;
+MvmSeg mvm_seg(const q35_q8f& W) { return MvmSeg{W.q, W.scale, W.cols, W.layout == Q35_KN_TILED ? 1 : 0}; }
+
+// f32 region of a layer call behind its other scratch: the rows between the launches, then the
+// gate and split-K partials of one row group
+struct MvmSizes {
+  size_t rows, aux, part;  // floats
+  size_t bytes() const { return align256(rows * 4) + align256(aux * 4) + align256(part * 4); }
+};
+MvmSizes mvm_sizes(const q35_dims& d, int B) {
+  const LayerDims L = ldims(d);
+  const size_t ldq = L.conv_dim + L.vdim, ldqkv = 2 * L.ah * L.hd + 2 * L.kvh * L.hd;
+  MvmSizes z;
+  z.rows = (size_t)B * std::max(ldq + 2 * L.nh, std::max(ldqkv, (size_t)L.F));
+  z.aux = mvm_aux_floats(B, L.H, L.nh);
+  z.part = std::max({mvm_part_floats(B, L.H, (int)ldq, false), mvm_part_floats(B, L.vdim, L.H, L.dv == 128),
+                     mvm_part_floats(B, L.H, (int)ldqkv, false), mvm_part_floats(B, L.ah * L.hd, L.H, false),
+                     mvm_part_floats(B, L.H, 2 * L.F, false), mvm_part_floats(B, L.F, L.H, false)});
+  return z;
+}
+size_t mvm_layer_bytes(const q35_dims& d, int B) { return B >= kMvmMin ? mvm_sizes(d, B).bytes() : 0; }
+
+// One projection of a layer call over all of its rows, kMvmRows at a time: c carries the first
+// row's pointers and the partials.
+int mvm_rows(MvmCall c, int B, hipStream_t st) {
+  for (int b0 = 0; b0 < B; b0 += kMvmRows) {
+    c.M = std::min(kMvmRows, B - b0);
+    const int rc = mvm_launch(c, st);
+    if (rc) return rc;
+    c.x += (size_t)kMvmRows * c.ldx;
+    c.y += (size_t)kMvmRows * c.ldy;
+    if (c.z) c.z += (size_t)kMvmRows * c.ldz;
+    if (c.bg) c.bg += (size_t)kMvmRows * 2 * c.aux_nh;
+  }
+  return Q35_OK;
+}
+
 size_t scratch_bytes(const q35_dims& d, int B, int tmax) {
   const LayerDims L = ldims(d);
   const size_t gdn = align256((size_t)B * L.vdim * 4);
@@ -127,7 +170,8 @@ size_t q35_q8_gemv_ws_bytes(int32_t M, q35_q8f W) {
   if (W.layout == Q35_KN_PANEL) return 0;
   if (W.layout == Q35_NK) return kCounterBytes;
   const int m = std::max(1, std::min<int>(M, 8));
-  return kCounterBytes + align256((size_t)m * W.cols * sizeof(fx_t));
+  return kCounterBytes + align256((size_t)m * W.cols * sizeof(fx_t)) +
+         (M >= kMvmGemvMin ? align256(mvm_part_floats(M, W.rows, W.cols, false) * sizeof(float)) : 0);
 }
 
 int q35_q8_gemv(const float* x, int32_t M, q35_q8f W, float* y, void* ws, size_t ws_bytes, void* stream) {
@@ -147,6 +191,15 @@ int q35_q8_gemv(const float* x, int32_t M, q35_q8f W, float* y, void* ws, size_t
     const int K = W.rows, N = W.cols;
     if (!ws || ws_bytes < q35_q8_gemv_ws_bytes(M, W)) return fail(Q35_E_WS, "q8_gemv: workspace too small");
     fx_t* acc = reinterpret_cast<fx_t*>(ws_scratch(ws));
+    if (M >= kMvmGemvMin && mvm_ok(x, K, K) && mvm_ok(y, N, K)) {  // matrix cores, up to 32 rows per launch
+      MvmCall c;
+      c.seg[0] = mvm_seg(W); c.nseg = 1; c.K = K; c.x = x; c.ldx = K; c.y = y; c.ldy = N;
+      c.part = reinterpret_cast<float*>(ws_scratch(ws) + align256((size_t)std::min(M, 8) * N * sizeof(fx_t)));
+      c.part_floats = mvm_part_floats(M, K, N, false);
+      c.clear = 1;  // (calls of other sizes place their zeroed sums there)
+      c.err = ws_counters(ws) + kWsErrWord;
+      return mvm_rows(c, M, S(stream));
+    }
     for (int m0 = 0; m0 < M; m0 += 8) {
       MvCall c;
       c.err = ws_counters(ws) + kWsErrWord;
@@ -230,7 +283,7 @@ int q35_workspace_status(void* ws, void* stream) {
 
 size_t q35_layer_ws_bytes(const q35_dims* d, int32_t B, int32_t tmax) {
   if (!d || B < 1) return 0;
-  return kCounterBytes + acc_bytes(*d, B) + scratch_bytes(*d, B, std::max(1, tmax));
+  return kCounterBytes + acc_bytes(*d, B) + scratch_bytes(*d, B, std::max(1, tmax)) + mvm_layer_bytes(*d, B);
 }
 
 int q35_gated_deltanet_decode(const q35_dims* d, const q35_gdn_weights* w, const float* x, int32_t B,
@@ -258,6 +311,31 @@ int q35_gated_deltanet_decode(const q35_dims* d, const q35_gdn_weights* w, const
   fx_t* y = ac.take<fx_t>((size_t)B * L.H);
   float* o = sc.take<float>((size_t)B * L.vdim);
   hipStream_t st = S(stream);
+  if (B >= kMvmMin && L.dv == 128 && L.nh <= 16 && (int64_t)B * L.nh <= kMaxCounters && mvm_ok(x, L.H, L.H) &&
+      mvm_ok(out, L.H, L.H) && (reinterpret_cast<uintptr_t>(w->norm_w) & 15) == 0) {
+    const MvmSizes z = mvm_sizes(*d, B);
+    Carver mc{ws_scratch(ws) + acc_bytes(*d, B) + scratch_bytes(*d, B, 1), z.bytes()};
+    float* qz = mc.take<float>(z.rows);
+    float* bg = qz + (size_t)B * ldq;
+    MvmCall c;  // in_proj_qkv | in_proj_z | in_proj_b,a
+    c.seg[0] = mvm_seg(w->in_proj_qkv); c.seg[1] = mvm_seg(w->in_proj_z); c.nseg = 2;
+    c.K = L.H; c.x = x; c.ldx = L.H; c.y = qz; c.ldy = ldq;
+    c.aux_wb = w->in_proj_b; c.aux_wa = w->in_proj_a; c.aux_nh = L.nh; c.a_log = w->a_log; c.dt_bias = w->dt_bias;
+    c.bg = bg; c.aux_part = mc.take<float>(z.aux);
+    c.part = mc.take<float>(z.part); c.part_floats = z.part;
+    c.err = ws_counters(ws) + kWsErrWord;
+    if ((rc = mvm_rows(c, B, st))) return rc;
+    GdnCall g;  // the step advances the conv state itself
+    g.qkv = qz; g.ld_qkv = ldq; g.bg = bg; g.ld_bg = 2 * L.nh;
+    g.conv_state = conv_state; g.conv_w = w->conv_w; g.S = rec_state; g.o = o; g.ld_o = L.vdim;
+    g.B = B; g.nh = L.nh; g.dk = L.dk; g.dv = L.dv; g.conv_k = d->conv_k; g.head_ctr = ws_counters(ws);
+    if ((rc = gdn_step_launch(g, st))) return rc;
+    MvmCall n;  // gated RMSNorm + out_proj
+    n.seg[0] = mvm_seg(w->out_proj); n.nseg = 1; n.K = L.vdim; n.x = o; n.ldx = L.vdim;
+    n.z = qz + L.conv_dim; n.ldz = ldq; n.pw = w->norm_w; n.eps = d->eps; n.y = out; n.ldy = L.H;
+    n.part = c.part; n.part_floats = z.part; n.err = c.err;
+    return mvm_rows(n, B, st);
+  }
   for (int b0 = 0; b0 < B; b0 += 8) {  // in_proj_qkv | in_proj_z | in_proj_b,a (text_modules.rs:497-508,569-576)
     MvCall c;
     c.err = ws_counters(ws) + kWsErrWord;
@@ -319,7 +397,19 @@ int q35_attention_decode(const q35_dims* d, const q35_attn_weights* w, const flo
   Carver sc{ws_scratch(ws) + abytes + (att_ws - kCounterBytes), ws_bytes - kCounterBytes - abytes - (att_ws - kCounterBytes)};
   float* att = sc.take<float>((size_t)B * ldo);
   hipStream_t st = S(stream);
-  for (int b0 = 0; b0 < B; b0 += 8) {  // q_proj | k_proj | v_proj (text_modules.rs:855-893)
+  const bool multi = B >= kMvmMin && mvm_ok(x, L.H, L.H) && mvm_ok(out, L.H, L.H);
+  const MvmSizes z = mvm_sizes(*d, multi ? B : 1);
+  Carver mc{ws_scratch(ws) + abytes + scratch_bytes(*d, B, tmax), multi ? z.bytes() : 0};
+  float* qkvr = multi ? mc.take<float>(z.rows) : nullptr;
+  MvmCall mv;
+  if (multi) {  // q_proj | k_proj | v_proj
+    mc.take<float>(z.aux);
+    mv.seg[0] = mvm_seg(w->q_proj); mv.seg[1] = mvm_seg(w->k_proj); mv.seg[2] = mvm_seg(w->v_proj); mv.nseg = 3;
+    mv.K = L.H; mv.x = x; mv.ldx = L.H; mv.y = qkvr; mv.ldy = LD;
+    mv.part = mc.take<float>(z.part); mv.part_floats = z.part; mv.err = ws_counters(ws) + kWsErrWord;
+    if ((rc = mvm_rows(mv, B, st))) return rc;
+  }
+  for (int b0 = 0; b0 < B && !multi; b0 += 8) {  // q_proj | k_proj | v_proj (text_modules.rs:855-893)
     MvCall c;
     c.err = ws_counters(ws) + kWsErrWord;
     c.K = L.H; c.M = std::min(8, B - b0); c.nseg = 3;
@@ -330,12 +420,23 @@ int q35_attention_decode(const q35_dims* d, const q35_attn_weights* w, const flo
     if ((rc = mv_kn_launch(c, st))) return rc;
   }
   AttnCall a;  // norms, RoPE, KV append, attention, gate (:860-936)
-  a.qg_f = qkv; a.ld_qg = LD; a.k_f = qkv + ldqg; a.v_f = qkv + ldqg + L.kvh * L.hd; a.ld_kv = LD;
+  a.ld_qg = LD; a.ld_kv = LD;
+  if (multi) {
+    a.qg = qkvr; a.k = qkvr + ldqg; a.v = qkvr + ldqg + L.kvh * L.hd;
+  } else {
+    a.qg_f = qkv; a.k_f = qkv + ldqg; a.v_f = qkv + ldqg + L.kvh * L.hd;
+  }
   a.qnw = w->q_norm; a.knw = w->k_norm; a.eps = d->eps;
   a.rcos = rope_cos; a.rsin = rope_sin; a.rot = d->rot_dim; a.kc = k_cache; a.vc = v_cache; a.tmax = tmax;
   a.pos = d_pos; a.out = att; a.ld_out = ldo; a.B = B; a.nh = L.ah; a.nkv = L.kvh; a.hd = L.hd;
   // the attention kernel takes [counters | partials]; its partials start right after the accumulators
   if ((rc = attn_launch_split(a, ws_counters(ws), ws_scratch(ws) + abytes, att_ws - kCounterBytes, st))) return rc;
+  if (multi) {
+    MvmCall o;
+    o.seg[0] = mvm_seg(w->o_proj); o.nseg = 1; o.K = ldo; o.x = att; o.ldx = ldo; o.y = out; o.ldy = L.H;
+    o.part = mv.part; o.part_floats = z.part; o.err = mv.err;
+    return mvm_rows(o, B, st);
+  }
   for (int b0 = 0; b0 < B; b0 += 8) {  // o_proj (:938-942)
     MvCall c;
     c.err = ws_counters(ws) + kWsErrWord;
@@ -366,6 +467,21 @@ int q35_mlp_decode(const q35_dims* d, const q35_mlp_weights* w, const float* x, 
   fx_t* gu = ac.take<fx_t>((size_t)B * 2 * L.F);
   fx_t* y = ac.take<fx_t>((size_t)B * L.H);
   hipStream_t st = S(stream);
+  if (B >= kMvmMin && mvm_ok(x, L.H, L.H) && mvm_ok(out, L.H, L.H)) {
+    const MvmSizes z = mvm_sizes(*d, B);
+    Carver mc{ws_scratch(ws) + acc_bytes(*d, B) + scratch_bytes(*d, B, 1), z.bytes()};
+    float* act = mc.take<float>(z.rows);
+    mc.take<float>(z.aux);
+    MvmCall c;  // gate_proj | up_proj, up * silu(gate)
+    c.seg[0] = mvm_seg(w->gate_proj); c.seg[1] = mvm_seg(w->up_proj); c.nseg = 2; c.K = L.H; c.x = x; c.ldx = L.H;
+    c.y = act; c.ldy = L.F; c.swiglu = 1;
+    c.part = mc.take<float>(z.part); c.part_floats = z.part; c.err = ws_counters(ws) + kWsErrWord;
+    if ((rc = mvm_rows(c, B, st))) return rc;
+    MvmCall n;  // down_proj
+    n.seg[0] = mvm_seg(w->down_proj); n.nseg = 1; n.K = L.F; n.x = act; n.ldx = L.F; n.y = out; n.ldy = L.H;
+    n.part = c.part; n.part_floats = z.part; n.err = c.err;
+    return mvm_rows(n, B, st);
+  }
   for (int b0 = 0; b0 < B; b0 += 8) {  // gate_proj | up_proj (text_modules.rs:1003-1004)
     MvCall c;
     c.err = ws_counters(ws) + kWsErrWord;

@@ -433,6 +433,39 @@ int mvp_launch(const int8_t* q, const float* s, int32_t K, int32_t N, const floa
 int fx_to_f32_launch(fx_t* acc, int64_t n, float* y, bool zero_after, hipStream_t st);
 int fx_zero_launch(fx_t* acc, int64_t n, hipStream_t st);
 
+// ------------------------------------------------------------------ multi-row matvec (mvm.hip)
+// y[m][n] = x~[m][:] . dequant(W)[:, n] for 2..32 rows over KN / KN_TILED weights on the f16 matrix
+// cores: the projection launch leaves K-split partials, the second kernel adds them (and applies
+// SwiGLU, or the DeltaNet gates' activations).
+constexpr int kMvmRows = 32, kMvmMaxSeg = 3;
+struct MvmSeg {
+  const int8_t* q = nullptr;
+  const float* s = nullptr;
+  int32_t N = 0;
+  int32_t tiled = 0;  // 1: Q35_KN_TILED (q[t][K][256], s[t][K][4])
+};
+struct MvmCall {
+  MvmSeg seg[kMvmMaxSeg];  // the outputs follow each other in a row of y
+  int32_t nseg = 0, K = 0, M = 0;
+  const float* x = nullptr; int32_t ldx = 0;  // rows 16-byte aligned
+  // gated RMSNorm over 128-wide heads (z set): x~ = pw * (x * rsqrt(mean(x^2) + eps)) * silu(z)
+  const float* z = nullptr; int32_t ldz = 0; const float* pw = nullptr; float eps = 1e-6f;
+  float* y = nullptr; int32_t ldy = 0;
+  int32_t swiglu = 0;  // y[m][j] = up * silu(gate): the outputs' second half times silu of the first
+  // DeltaNet gates: bg[m] = [beta | g] from x . in_proj_b | x . in_proj_a (aux_nh heads <= 16)
+  const float* aux_wb = nullptr; const float* aux_wa = nullptr; int32_t aux_nh = 0;
+  const float* a_log = nullptr; const float* dt_bias = nullptr; float* bg = nullptr;
+  float* aux_part = nullptr;                      // mvm_aux_floats
+  float* part = nullptr; size_t part_floats = 0;  // mvm_part_floats
+  int32_t clear = 0;  // zero the partials behind the call (a workspace shared by calls of other sizes)
+  uint32_t* err = nullptr;                        // receives kWsErrRange
+};
+size_t mvm_part_floats(int32_t M, int32_t K, int32_t N, bool gated);
+size_t mvm_aux_floats(int32_t M, int32_t K, int32_t nh);
+// The rows and K mvm_launch takes (else the one-row kernel's row groups do).
+bool mvm_ok(const float* x, int32_t ldx, int32_t K);
+int mvm_launch(const MvmCall& c, hipStream_t st);
+
 // ------------------------------------------------------------------ Q8F GEMM (prompt projections)
 // Y[m][n] (+)= X[m][:] . dequant(W)[:, n] on the fp32 matrix cores; up to kGemmMaxSeg weight
 // matrices over the same X, each writing its own columns of Y.

@@ -1,0 +1,88 @@
+"""The multi-row matrix-core matvec (q8_gemv from 2 rows, layer calls from 2 sequences) against
+float64: edges of its row tiles (16, 32, 33 rows), of its column blocks and tiles (64, 320: a partial
+256-column tile), of its K ranges (64: one short wave; 160: a range that ends inside a block), both
+layouts, and one workspace shared by calls of different sizes and row counts.
+
+Bound: the products are exact and the sums f32 over K <= 6144 (a few 2^-24 per partial sum, random
+signs: seen 1e-7 to 3e-7); 2e-6 is taken."""
+import numpy as np
+import pytest
+import torch
+
+import q35
+from conftest import rel_l2
+from gpu_util import dev, host, normal, q8, q8_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("layout", ["kn", "tiled"])
+@pytest.mark.parametrize("K,N,M", [(64, 64, 2), (160, 320, 3), (2048, 512, 16), (2048, 6144, 17), (6144, 2048, 32),
+                                   (2048, 2048, 33), (96, 192, 64)])
+def test_q8_gemv_rows(K, N, M, layout):
+    print(f"[gemv rows] K={K} N={N} M={M} {layout}", flush=True)
+    W = q8(400 + K + N, K, N)
+    x = normal(401 + M, (M, K)) * np.exp(normal(402, (M, 1))).astype(np.float32)
+    Wd = q8_dev(W, q35.Q35_KN)
+    y = host(q35.q8_gemv(dev(x), Wd.tiled() if layout == "tiled" else Wd))
+    ref = x.astype(np.float64) @ W.dequant()
+    for m in range(M):
+        assert rel_l2(y[m], ref[m]) <= 2e-6, m
+
+
+def test_q8_gemv_rows_share_a_workspace_with_other_sizes():
+    """Row counts and widths alternate on the one workspace of q8_gemv: every call's sums start from
+    zero whatever ran before, including the one-row kernel's fixed-point words."""
+    for K, N, M in [(2048, 512, 8), (2048, 8192, 1), (2048, 6144, 32), (64, 8192, 1), (2048, 512, 1), (2048, 2048, 5)]:
+        W = q8(420, K, N)
+        x = normal(421 + M, (M, K))
+        y = host(q35.q8_gemv(dev(x), q8_dev(W, q35.Q35_KN)))
+        assert rel_l2(y, x.astype(np.float64) @ W.dequant()) <= 2e-6, (K, N, M)
+
+
+def test_q8_gemv_rows_unaligned_input_and_magnitudes():
+    """Rows that start 4 bytes past a 16-byte boundary take the one-row kernel; rows of zeros and of
+    magnitudes 1e-20 to 1e6 keep their relative precision where the fixed-point sums would not."""
+    K, N, M = 2048, 1024, 6
+    W = q8(430, K, N)
+    x = normal(431, (M, K))
+    ref = x.astype(np.float64) @ W.dequant()
+    buf = torch.empty(M * K + 1, device="cuda")
+    buf[1:] = dev(x).reshape(-1)
+    xu = buf[1:].view(M, K)
+    assert xu.data_ptr() % 16 != 0
+    Wd = q8_dev(W, q35.Q35_KN)
+    assert rel_l2(host(q35.q8_gemv(xu, Wd)), ref) <= 2e-6
+    mag = np.array([1e-20, 1e-6, 1.0, 0.0, 1e3, 1e6], np.float32)
+    y = host(q35.q8_gemv(dev(x * mag[:, None]), Wd))
+    for m in range(M):
+        if mag[m] == 0:
+            np.testing.assert_array_equal(y[m], 0.0)
+        else:
+            assert rel_l2(y[m], ref[m] * float(mag[m])) <= 2e-6, m
+
+
+@pytest.mark.parametrize("B", [2, 33])
+def test_layers_in_row_groups(B):
+    """MLP and attention over one row group and a second one (33 = 32 + 1 rows): each row as by itself."""
+    d = q35.dims_2b()
+    H, nh, nkv, hd = d.hidden, d.attn_heads, d.kv_heads, d.head_dim
+    x = dev(normal(440, (B, H)))
+    mlp = q35.MLP(d, *(q8_dev(q8(441 + i, *s), q35.Q35_KN).tiled() for i, s in
+                       enumerate([(H, d.ffn), (H, d.ffn), (d.ffn, H)])))
+    att = q35.Attention(d, *(q8_dev(q8(445 + i, *s), q35.Q35_KN) for i, s in
+                             enumerate([(H, nh * hd * 2), (H, nkv * hd), (H, nkv * hd), (nh * hd, H)])),
+                        dev(normal(450, (hd,), 0.1)), dev(normal(451, (hd,), 0.1)))
+    tmax = 40
+    cs, sn = q35.rope_tables(d, tmax)
+    kc, vc = normal(452, (B, nkv, tmax, hd)), normal(453, (B, nkv, tmax, hd))
+    pos = (np.arange(B) % tmax).astype(np.int32)
+    kd, vd = dev(kc), dev(vc)
+    out_m = host(mlp.forward(x, check=True))
+    out_a = host(att.forward(x, kd, vd, dev(pos), dev(cs), dev(sn)))
+    for b in range(B):
+        k1, v1 = dev(kc[b:b + 1]), dev(vc[b:b + 1])
+        assert rel_l2(out_m[b], host(mlp.forward(x[b:b + 1]))[0]) <= 3e-6, b
+        one = host(att.forward(x[b:b + 1], k1, v1, dev(pos[b:b + 1]), dev(cs), dev(sn)))
+        assert rel_l2(out_a[b], one[0]) <= 3e-6, b
+        assert rel_l2(host(kd[b]), host(k1[0])) <= 2e-6 and rel_l2(host(vd[b]), host(v1[0])) <= 2e-6
