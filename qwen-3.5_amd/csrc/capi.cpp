@@ -684,8 +684,10 @@ int q35_gated_delta_rule_prefill(const float* mixed_qkv, int32_t T, int32_t ld_q
   GdnPrefill g;
   g.raw = mixed_qkv; g.ld_raw = ld_qkv; g.conv_state = conv_state; g.conv_state_out = conv_state; g.conv_w = conv_w;
   g.bg = beta_g; g.ld_bg = 2 * lin_heads; g.scr = static_cast<float*>(ws); g.S = rec_state; g.out = core_out;
-  g.ld_out = lin_heads * lin_dv; g.T = T; g.nh = lin_heads; g.key_dim = key_dim;
-  g.nchunk = (T + kGdnChunk - 1) / kGdnChunk; g.qscale = powf((float)lin_dk, -0.5f);
+  g.ld_out = lin_heads * lin_dv; g.nh = lin_heads; g.key_dim = key_dim;
+  PfSeqs sq;
+  sq.add(T, 0, 0, kGdnChunk, 1);
+  g.sq = pf_arg(sq, nullptr); g.qscale = powf((float)lin_dk, -0.5f);
   return gdn_prefill_launch(g, S(stream));
 }
 
@@ -709,7 +711,11 @@ int q35_attention_core_prefill(const q35_dims* d, const float* q_gate, int32_t l
   AttnPrefill a;
   a.qg = q_gate; a.ld_qg = ld_qg; a.k = k_new; a.v = v_new; a.ld_kv = kv_ld; a.qnw = q_norm; a.knw = k_norm;
   a.eps = d->eps; a.rcos = rope_cos; a.rsin = rope_sin; a.rot = d->rot_dim; a.kc = k_cache; a.vc = v_cache;
-  a.tmax = tmax; a.p0 = p0; a.T = T; a.nh = d->attn_heads; a.nkv = d->kv_heads; a.qbuf = static_cast<float*>(ws);
+  a.tmax = tmax; a.nh = d->attn_heads; a.nkv = d->kv_heads;
+  PfSeqs sq;
+  if (T >= 1) sq.add(T, p0, 0, kGdnChunk, pf_attn_tile(a.nh, a.nkv));
+  a.sq = pf_arg(sq, nullptr);
+  a.qbuf = static_cast<float*>(ws);
   a.out = out; a.ld_out = d->attn_heads * d->head_dim; a.scale = (float)(1.0 / std::sqrt((double)d->head_dim));
   return attn_prefill_launch(a, S(stream));
 }

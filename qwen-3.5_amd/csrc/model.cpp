@@ -289,9 +289,7 @@ SeqView model_view(q35_model* m) {
     v.kc.push_back(L.kc);
     v.vc.push_back(L.vc);
   }
-  v.token = m->token;
-  v.pos = m->pos;
-  v.hist = m->hist;
+  v.prompt = m->prompt;
   v.tmax = m->tmax;
   return v;
 }
@@ -316,7 +314,7 @@ int ensure_prefill(q35_model* m, hipStream_t st) {
   const int cap = std::min(kPrefillCap, (m->tmax + kGdnChunk - 1) / kGdnChunk * kGdnChunk);
   const int ldy = std::max({conv_dim + vdim, ah * hd * 2 + 2 * kvh * hd, 2 * F});
   const int lda = std::max({vdim, ah * hd, F});
-  const size_t nchunk = (size_t)cap / kGdnChunk;
+  const size_t nchunk = (size_t)cap / kGdnChunk + kPfExtraChunks;
   if ((rc = dev_alloc_t(m, "prefill_x", (size_t)cap * H, &m->pf_x)) ||
       (rc = dev_alloc_t(m, "prefill_xn", (size_t)cap * H, &m->pf_xn)) ||
       (rc = dev_alloc_t(m, "prefill_y", (size_t)cap * ldy, &m->pf_y)) ||
@@ -327,7 +325,8 @@ int ensure_prefill(q35_model* m, hipStream_t st) {
       (rc = dev_alloc_t(m, "prefill_scratch", (size_t)nh * nchunk * kGdnScratchPerChunk, &m->pf_scr)) ||
       (rc = dev_alloc_t(m, "prefill_partials", gemm_part_floats(cap, H), &m->pf_part)) ||
       (rc = dev_alloc_t(m, "prefill_gemm_aux", gemm_aux_floats(cap), &m->pf_aux)) ||
-      (rc = dev_alloc_t(m, "prefill_act_max", (size_t)cap, &m->pf_act_max)))
+      (rc = dev_alloc_t(m, "prefill_act_max", (size_t)cap, &m->pf_act_max)) ||
+      (rc = dev_alloc_t(m, "prefill_seqs", 1, &m->pf_seqs)))
     return rc;
   // gate | up interleaved by 64-column block for the fused SwiGLU: an MB copy keeps each column
   // block's records (K * 64 bytes) and scales (K floats) contiguous, so the two copies are
@@ -358,17 +357,31 @@ int ensure_prefill(q35_model* m, hipStream_t st) {
   return Q35_OK;
 }
 
-// One pass over T <= pf_cap prompt tokens ids[0..T) at positions p0..p0+T-1: every layer on all
-// T rows (GEMM projections on the matrix cores, conv + chunked delta rule, causal attention),
-// then the final norm and the tied lm_head for the last row only (the only logits the greedy
-// loop reads, main.rs:93-95), whose argmax goes to the token slot and hist[p0+T-1].
-int prefill_pass(q35_model* m, const SeqView& v, const int32_t* ids, int T, int p0, hipStream_t st) {
+bool prefill_add(const q35_model* m, PfSeqs& sq, int rows, int p0, int slot) {
+  if (sq.n == kPfSeqs || sq.row0[sq.n] + rows > m->pf_cap ||
+      sq.chunk0[sq.n] + (rows + kGdnChunk - 1) / kGdnChunk > m->pf_cap / kGdnChunk + kPfExtraChunks)
+    return false;
+  sq.add(rows, p0, slot, kGdnChunk, pf_attn_tile(m->d.attn_heads, m->d.kv_heads));
+  return true;
+}
+
+// One pass over the prompt rows of one or more sequences: every layer on all rows (GEMM projections
+// on the matrix cores, which read each weight once for all of them; conv + chunked delta rule and
+// causal attention per sequence).
+int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t st) {
   const q35_dims& d = m->d;
+  for (int i = 0; i < seqs.n; ++i)
+    if (seqs.p0[i] < 0 || (int64_t)seqs.p0[i] + seqs.row0[i + 1] - seqs.row0[i] > v.tmax)
+      return fail(Q35_E_SHAPE, "prompt pass: positions past tmax");
+  // (from pageable memory: the copy has taken the table when the call returns)
+  if (seqs.n > 1) Q35_HIP_TRY(hipMemcpyAsync(m->pf_seqs, &seqs, sizeof(seqs), hipMemcpyHostToDevice, st));
+  const PfArg sq = pf_arg(seqs, m->pf_seqs);
+  const int T = sq.rows;
   const int H = d.hidden, F = d.ffn, nh = d.lin_heads, vdim = nh * d.lin_dv, key_dim = nh * d.lin_dk;
   const int conv_dim = 2 * key_dim + vdim, ah = d.attn_heads, kvh = d.kv_heads, hd = d.head_dim;
   const int LDY = m->pf_ldy;
   int rc;
-  if ((rc = embed_launch(m->embed.q, m->embed.s, d.vocab, H, ids, T, m->pf_x, st))) return rc;
+  if ((rc = embed_seqs_launch(m->embed.q, m->embed.s, H, v.prompt, v.tmax, sq, m->pf_x, st))) return rc;
   // projections on the f16 matrix cores from the MB copies of the weights
   auto seg = [](const q35_model::Q8& w, const q35_model::Mb& mb, float* y, int ldy) {
     return GemmSeg{mb.q, mb.s, y, w.cols, Q35_KN_MB, ldy, mb.smax};
@@ -396,8 +409,8 @@ int prefill_pass(q35_model* m, const SeqView& v, const int32_t* ids, int T, int 
       GdnPrefill gp;
       gp.raw = m->pf_y; gp.ld_raw = LDY; gp.conv_state = v.conv[l]; gp.conv_state_out = v.conv[l];
       gp.conv_w = L.conv_w; gp.bg = m->pf_bg; gp.ld_bg = 2 * nh; gp.scr = m->pf_scr; gp.S = v.rec[l];
-      gp.out = m->pf_core; gp.ld_out = vdim; gp.T = T; gp.nh = nh; gp.key_dim = key_dim;
-      gp.nchunk = (T + kGdnChunk - 1) / kGdnChunk; gp.qscale = powf((float)d.lin_dk, -0.5f);
+      gp.out = m->pf_core; gp.ld_out = vdim; gp.nh = nh; gp.key_dim = key_dim; gp.sq = sq;
+      gp.qscale = powf((float)d.lin_dk, -0.5f);
       if ((rc = gdn_prefill_launch(gp, st))) return rc;
       if ((rc = gated_norm_rows_launch(m->pf_core, vdim, m->pf_y + conv_dim, LDY, L.norm_w, T, nh, d.eps, m->pf_a, vdim, st,
                                        m->pf_aux)))
@@ -420,7 +433,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const int32_t* ids, int T, int 
       AttnPrefill ap;
       ap.qg = m->pf_y; ap.ld_qg = LDY; ap.k = m->pf_y + qw; ap.v = m->pf_y + qw + kvw; ap.ld_kv = LDY;
       ap.qnw = L.q_norm; ap.knw = L.k_norm; ap.eps = d.eps; ap.rcos = m->rope_cos; ap.rsin = m->rope_sin;
-      ap.rot = d.rot_dim; ap.kc = v.kc[l]; ap.vc = v.vc[l]; ap.tmax = v.tmax; ap.p0 = p0; ap.T = T; ap.nh = ah;
+      ap.rot = d.rot_dim; ap.kc = v.kc[l]; ap.vc = v.vc[l]; ap.tmax = v.tmax; ap.sq = sq; ap.nh = ah;
       ap.nkv = kvh; ap.qbuf = m->pf_q; ap.out = m->pf_a; ap.ld_out = ah * hd;
       ap.scale = (float)(1.0 / sqrt((double)hd));
       if ((rc = attn_prefill_launch(ap, st))) return rc;
@@ -451,16 +464,25 @@ int prefill_pass(q35_model* m, const SeqView& v, const int32_t* ids, int T, int 
     dn.part = m->pf_part; dn.part_floats = gemm_part_floats(m->pf_cap, d.hidden); dn.aux = m->pf_aux; dn.amax = m->pf_act_max;
       if ((rc = gemm_launch(dn, st))) return rc;
   }
-  if ((rc = store_i32_launch(v.pos, p0 + T - 1, st))) return rc;
+  return Q35_OK;
+}
+
+namespace {
+
+// The final norm and the tied lm_head of the pass's last row only (the only logits the greedy loop
+// reads, main.rs:93-95); its argmax goes to the token slot and hist[pos].
+int prefill_head(q35_model* m, int T, int pos, hipStream_t st) {
+  const q35_dims& d = m->d;
+  const int H = d.hidden;
+  const int rc = store_i32_launch(m->pos, pos, st);
+  if (rc) return rc;
   NkCall n;
   n.q = m->embed.q; n.s = m->embed.s; n.N = d.vocab; n.K = H; n.M = 1;
   n.x = m->pf_x + (size_t)(T - 1) * H; n.ldx = H; n.y = m->logits; n.ldy = d.vocab; n.pro = PRO_RMS;
   n.pw = m->final_norm; n.eps = d.eps;
-  n.argmax_out = v.token; n.pos_inc = v.pos; n.hist = v.hist;
+  n.argmax_out = m->token; n.pos_inc = m->pos; n.hist = m->hist;
   return nk_launch(n, m->ws, m->ws_bytes, st);
 }
-
-namespace {
 
 // The n prompt ids already in m->prompt[host_pos..) through the prompt path, in passes.
 int prefill(q35_model* m, int n, hipStream_t st) {
@@ -469,9 +491,12 @@ int prefill(q35_model* m, int n, hipStream_t st) {
   if ((int64_t)m->host_pos + n > m->tmax) return fail(Q35_E_SHAPE, "model_prefill: tmax too small");
   for (int done = 0; done < n;) {
     const int T = std::min(m->pf_cap, n - done);
-    if ((rc = prefill_pass(m, model_view(m), m->prompt + m->host_pos, T, m->host_pos, st))) return rc;
+    PfSeqs sq;
+    if (!prefill_add(m, sq, T, m->host_pos, 0)) return fail(Q35_E_SHAPE, "model_prefill: pass too large");
+    if ((rc = prefill_pass(m, model_view(m), sq, st))) return rc;
     m->host_pos += T;
     done += T;
+    if ((rc = prefill_head(m, T, m->host_pos - 1, st))) return rc;
   }
   return Q35_OK;
 }

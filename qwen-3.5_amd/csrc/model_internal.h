@@ -58,6 +58,7 @@ struct q35_model {
   int pf_cap = 0, pf_ldy = 0, pf_lda = 0;
   float *pf_x = nullptr, *pf_xn = nullptr, *pf_y = nullptr, *pf_a = nullptr, *pf_core = nullptr;
   float *pf_bg = nullptr, *pf_q = nullptr, *pf_scr = nullptr, *pf_part = nullptr, *pf_aux = nullptr;
+  q35::PfSeqs* pf_seqs = nullptr;  // device copy of a pass's sequence table
   float* pf_act_max = nullptr;  // row maxima of the SwiGLU rows (down_proj's input)
   // batched decode (allocated on first use): every projection again in the MB layout of the
   // matrix-core batch kernels (q[N/64][K/16][64][16], scale[N/64][K])
@@ -88,18 +89,21 @@ int dev_alloc_t(q35_model* m, const std::string& name, size_t n, T** out) {
 }
 hipStream_t pick(q35_model* m, void* s);
 
-// Where a prompt pass reads and writes one sequence's state: per-layer caches (null where a layer
-// has none), the token slot, the position and the history (positions 0 .. tmax-1).
+// The state a prompt pass reads and writes: per-layer caches (null where a layer has none) of slot 0,
+// the other slots' behind it, and the prompt ids prompt[slot * tmax + position].
 struct SeqView {
   std::vector<float*> conv, rec, kc, vc;
-  int32_t *token = nullptr, *pos = nullptr, *hist = nullptr;
+  const int32_t* prompt = nullptr;
   int32_t tmax = 0;
 };
 SeqView model_view(q35_model* m);
 // Allocates the prompt-path scratch and builds the MB weight copies on first use.
 int ensure_prefill(q35_model* m, hipStream_t st);
-// One prompt pass of T <= m->pf_cap tokens (device ids) at positions p0.. of sequence v.
-int prefill_pass(q35_model* m, const SeqView& v, const int32_t* ids, int T, int p0, hipStream_t st);
+constexpr int kPfExtraChunks = 16;  // chunk slots beyond pf_cap / 64, for sequences with a partial last chunk
+// Appends `rows` rows at position p0 of a slot to a pass; false when they do not fit it.
+bool prefill_add(const q35_model* m, PfSeqs& sq, int rows, int p0, int slot);
+// One prompt pass over sq's rows (at most m->pf_cap): their residual rows are left in m->pf_x.
+int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t st);
 // Builds the MB-layout copies of the projection weights on first use.
 int ensure_mb(q35_model* m, hipStream_t st);
 

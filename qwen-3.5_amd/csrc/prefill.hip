@@ -319,9 +319,12 @@ __global__ __launch_bounds__(kPP) void gdn_chunk_prep_kernel(const GdnPrefill a)
   __shared__ float cum[kC], bet[kC], ecum[kC];
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int c = blockIdx.x % a.nchunk, h = blockIdx.x / a.nchunk;
-  const int t0 = c * kC;
-  float* scr = a.scr + ((int64_t)h * a.nchunk + c) * kGdnScratchPerChunk;
+  const int nchunk = a.sq.chunks, c = blockIdx.x % nchunk, h = blockIdx.x / nchunk;
+  const PfSeq sq = pf_seq<&PfSeqs::chunk0>(a.sq, c);
+  const int tb = sq.tb, te = tb + sq.T;  // the sequence's rows
+  const int t0 = tb + (c - sq.cbeg) * kC;
+  const float* conv_state = a.conv_state + (int64_t)sq.slot * (2 * a.key_dim + a.nh * kDk) * 3;
+  float* scr = a.scr + ((int64_t)h * nchunk + c) * kGdnScratchPerChunk;
 
   // causal conv (cached state prepended) + SiLU: one channel of the head's 3 x 128 per thread
   // pass, a sliding window of the last three inputs in registers
@@ -337,27 +340,27 @@ __global__ __launch_bounds__(kPP) void gdn_chunk_prep_kernel(const GdnPrefill a)
 #pragma unroll
       for (int u = 0; u < 3; ++u) {
         const int tt = t0 - 3 + u;
-        xw[u] = tt >= 0 ? a.raw[(int64_t)tt * a.ld_raw + ch] : a.conv_state[(int64_t)ch * 3 + 3 + tt];
+        xw[u] = tt >= tb ? a.raw[(int64_t)tt * a.ld_raw + ch] : conv_state[(int64_t)ch * 3 + 3 + tt - tb];
       }
       x0 = xw[0]; x1 = xw[1]; x2 = xw[2];
     }
     // all of the chunk's inputs of the channel in flight at once (rows clamped, masked below)
     float xv[kC];
 #pragma unroll
-    for (int u = 0; u < kC; ++u) xv[u] = a.raw[(int64_t)min(t0 + u, a.T - 1) * a.ld_raw + ch];
+    for (int u = 0; u < kC; ++u) xv[u] = a.raw[(int64_t)min(t0 + u, te - 1) * a.ld_raw + ch];
 #pragma unroll
     for (int u = 0; u < kC; ++u) {
       const int t = t0 + u;
-      const float xin = t < a.T ? xv[u] : 0.f;
+      const float xin = t < te ? xv[u] : 0.f;
       const float y = ((w0 * x0 + w1 * x1) + w2 * x2) + w3 * xin;
-      dst[u][cc] = t < a.T ? silu_f(y) : 0.f;
+      dst[u][cc] = t < te ? silu_f(y) : 0.f;
       x0 = x1; x1 = x2; x2 = xin;
     }
   }
   if (tid < kC) {
     const int t = t0 + tid;
-    bet[tid] = t < a.T ? a.bg[(int64_t)t * a.ld_bg + h] : 0.f;
-    cum[tid] = t < a.T ? a.bg[(int64_t)t * a.ld_bg + a.nh + h] : 0.f;  // g for now
+    bet[tid] = t < te ? a.bg[(int64_t)t * a.ld_bg + h] : 0.f;
+    cum[tid] = t < te ? a.bg[(int64_t)t * a.ld_bg + a.nh + h] : 0.f;  // g for now
   }
   for (int e = tid; e < kC * kC; e += kPP) U[e >> 6][e & 63] = 0.f;
   __syncthreads();
@@ -493,21 +496,22 @@ __global__ __launch_bounds__(kST) void gdn_chunk_state_kernel(const GdnPrefill a
   __shared__ __align__(16) mfma_f4 RedO[4][64];    // upper halves' output partials
 
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c16 = l & 15, g = l >> 4;
-  const int sl = blockIdx.x % kNsl, h = blockIdx.x / kNsl;
-  const int c0 = sl * kSl;
-  float* S = a.S + (int64_t)h * kDk * kDk;
+  const int sl = blockIdx.x % kNsl, h = (blockIdx.x / kNsl) % a.nh;
+  const PfSeq sq = pf_nth(a.sq, blockIdx.x / (kNsl * a.nh));
+  const int c0 = sl * kSl, tb = sq.tb, T = sq.T, nchunk = sq.nchunk;
+  float* S = a.S + ((int64_t)sq.slot * a.nh + h) * kDk * kDk;
   // the new conv state of the head's channels: the last 3 inputs (older ones from the old state
   // when the prompt is shorter than 3); the prep launch has read the old state already
   if (sl == 0 && a.conv_state_out) {
     for (int e = tid; e < 3 * kDk; e += kST) {
       const int part = e >> 7, jj = e & 127;
       const int ch = part == 0 ? h * kDk + jj : (part == 1 ? a.key_dim + h * kDk + jj : 2 * a.key_dim + h * kDk + jj);
-      float* st = a.conv_state_out + (int64_t)ch * 3;
+      float* st = a.conv_state_out + ((int64_t)sq.slot * (2 * a.key_dim + a.nh * kDk) + ch) * 3;
       float n[3];
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        const int src = k + a.T;  // index into [old s0, s1, s2, x_0, x_1, ...]
-        n[k] = src < 3 ? st[src] : a.raw[(int64_t)(src - 3) * a.ld_raw + ch];
+        const int src = k + T;  // index into [old s0, s1, s2, x_0, x_1, ...]
+        n[k] = src < 3 ? st[src] : a.raw[(int64_t)(tb + src - 3) * a.ld_raw + ch];
       }
       st[0] = n[0]; st[1] = n[1]; st[2] = n[2];
     }
@@ -520,7 +524,7 @@ __global__ __launch_bounds__(kST) void gdn_chunk_state_kernel(const GdnPrefill a
   }
   const int rt = w & 3, kh = w >> 2;  // chunk-row tile and key-row half of the wave
   auto load_ops = [&](int c, StateOps& o) {
-    const float* scr = a.scr + ((int64_t)h * a.nchunk + c) * kGdnScratchPerChunk;
+    const float* scr = a.scr + ((int64_t)h * a.sq.chunks + sq.cbeg + c) * kGdnScratchPerChunk;
     const float* kr = scr + kScrKcd + (rt * 2 + kh) * 4 * 256 + 4 * l;
     const float* qr = scr + kScrQe + (rt * 2 + kh) * 4 * 256 + 4 * l;
     const float* ir = scr + kScrIntra + rt * 4 * 256 + 4 * l;
@@ -543,8 +547,8 @@ __global__ __launch_bounds__(kST) void gdn_chunk_state_kernel(const GdnPrefill a
   load_ops(0, cur);
   __syncthreads();
   int sb = 0;  // state buffer of the current chunk
-  for (int c = 0; c < a.nchunk; ++c) {
-    if (c + 1 < a.nchunk) load_ops(c + 1, nxt);
+  for (int c = 0; c < nchunk; ++c) {
+    if (c + 1 < nchunk) load_ops(c + 1, nxt);
     // v_new: rows 16 rt + 4 g + r, column c16; key rows [64 kh, 64 kh + 64)
     {
       mfma_f4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -599,7 +603,7 @@ __global__ __launch_bounds__(kST) void gdn_chunk_state_kernel(const GdnPrefill a
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int t = c * kC + 16 * rt + 4 * g + r;
-          if (t < a.T) a.out[(int64_t)t * a.ld_out + h * kDk + c0 + c16] = (oacc[r] + up[r]) + pacc[r];
+          if (t < T) a.out[(int64_t)(tb + t) * a.ld_out + h * kDk + c0 + c16] = (oacc[r] + up[r]) + pacc[r];
         }
       }
     }
@@ -644,7 +648,8 @@ __global__ __launch_bounds__(kPT) void attn_prefill_prep_kernel(const AttnPrefil
   __shared__ float xs[kHdP];
   const int t = blockIdx.x / (a.nh + a.nkv), slot = blockIdx.x % (a.nh + a.nkv);
   const int tid = threadIdx.x;
-  const int pos = a.p0 + t;
+  const PfSeq sq = pf_seq<&PfSeqs::row0>(a.sq, t);
+  const int pos = sq.p0 + t - sq.tb;
   const float* src;
   const float* nw;
   if (slot < a.nh) {
@@ -669,7 +674,7 @@ __global__ __launch_bounds__(kPT) void attn_prefill_prep_kernel(const AttnPrefil
     a.qbuf[((int64_t)t * a.nh + slot) * kHdP + tid] = y;
   } else {
     const int g = slot - a.nh;
-    const int64_t row = ((int64_t)g * a.tmax + pos) * kHdP;
+    const int64_t row = (((int64_t)sq.slot * a.nkv + g) * a.tmax + pos) * kHdP;
     a.kc[row + tid] = y;
     a.vc[row + tid] = a.v[(int64_t)t * a.ld_kv + (int64_t)g * kHdP + tid];
   }
@@ -695,18 +700,21 @@ __global__ __launch_bounds__(kAT, 1) void attn_prefill_kernel(const AttnPrefill 
   __shared__ float Mw[kAW][kRows], Lw[kAW][kRows];
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c16 = l & 15, g = l >> 4;
   const int rep = a.nh / a.nkv, QT = kRows / rep;
-  const int qt = blockIdx.x / a.nkv, gk = blockIdx.x % a.nkv;
-  const int t = qt * QT + c16 / rep;  // the lane's query row c16: token t
-  const int lim = a.p0 + min(t, a.T - 1);  // last key row c16 may see (rows past T are discarded)
-  const int tmax_blk = min(a.T, (qt + 1) * QT) - 1;
-  const int nkeys = a.p0 + tmax_blk + 1;
+  const int gk = blockIdx.x % a.nkv, tile = blockIdx.x / a.nkv;
+  const PfSeq sq = pf_seq<&PfSeqs::tile0>(a.sq, tile);
+  const int qt = tile - sq.tile0, tb = sq.tb, T = sq.T, p0 = sq.p0;
+  const int t = qt * QT + c16 / rep;  // the lane's query row c16: token t of the sequence
+  const int lim = p0 + min(t, T - 1);  // last key row c16 may see (rows past T are discarded)
+  const int tmax_blk = min(T, (qt + 1) * QT) - 1;
+  const int nkeys = p0 + tmax_blk + 1;
   for (int e = tid; e < kRows * kHdP / 4; e += kAT) {
     const int r = e >> 6, d = (e & 63) * 4;
-    const int tr = min(qt * QT + r / rep, a.T - 1), hr = gk * rep + r % rep;
+    const int tr = tb + min(qt * QT + r / rep, T - 1), hr = gk * rep + r % rep;
     *(q35_f32x4*)&Qs[r][d] = *(const q35_f32x4*)(a.qbuf + ((int64_t)tr * a.nh + hr) * kHdP + d);
   }
-  const float* Kg = a.kc + (int64_t)gk * a.tmax * kHdP;
-  const float* Vg = a.vc + (int64_t)gk * a.tmax * kHdP;
+  const int64_t cache = ((int64_t)sq.slot * a.nkv + gk) * a.tmax * kHdP;
+  const float* Kg = a.kc + cache;
+  const float* Vg = a.vc + cache;
   float (*Kt)[kKvLd] = KV[w][0];
   float (*Vt)[kKvLd] = KV[w][1];
   q35_f32x4 nk[16], nv[16];  // the next tile: key row u, dims 4 l .. 4 l + 3
@@ -784,8 +792,9 @@ __global__ __launch_bounds__(kAT, 1) void attn_prefill_kernel(const AttnPrefill 
   }
   __syncthreads();
   const int q = tid >> 4, d0 = (tid & 15) * 16;
-  const int tq = qt * QT + q / rep, hq = gk * rep + q % rep;
-  if (tq >= a.T) return;
+  const int hq = gk * rep + q % rep;
+  if (qt * QT + q / rep >= T) return;
+  const int tq = tb + qt * QT + q / rep;
   float M = Mw[0][q];
 #pragma unroll
   for (int ww = 1; ww < kAW; ++ww) M = fmaxf(M, Mw[ww][q]);
@@ -808,6 +817,23 @@ __global__ __launch_bounds__(kAT, 1) void attn_prefill_kernel(const AttnPrefill 
   }
 }
 
+// Block t: the embedding row of prompt row t (kernels.rs:15-45).
+__global__ __launch_bounds__(kPT) void embed_seqs_kernel(const int8_t* q, const float* s, int D, const int32_t* prompt,
+                                                         int ldp, const PfArg sq, float* x) {
+  const int t = blockIdx.x;
+  const PfSeq s1 = pf_seq<&PfSeqs::row0>(sq, t);
+  const int64_t tok = prompt[(int64_t)s1.slot * ldp + s1.p0 + t - s1.tb];
+  for (int k = threadIdx.x; k < D; k += kPT) x[(int64_t)t * D + k] = (float)q[tok * D + k] * s[tok * (D / 64) + (k >> 6)];
+}
+
+__global__ __launch_bounds__(kPT) void last_rows_kernel(const float* x, int ldx, int D, const PfArg sq, float* h,
+                                                        int32_t* pos) {
+  const PfSeq s = pf_nth(sq, blockIdx.x);
+  const int t = s.tb + s.T - 1, slot = s.slot;
+  for (int k = threadIdx.x; k < D; k += kPT) h[(int64_t)slot * D + k] = x[(int64_t)t * ldx + k];
+  if (threadIdx.x == 0) pos[slot] = s.p0 + s.T - 1;
+}
+
 __global__ void store_i32_kernel(int32_t* p, int32_t v) {
   if (threadIdx.x == 0) *p = v;
 }
@@ -816,6 +842,19 @@ __global__ void store_i32_kernel(int32_t* p, int32_t v) {
 
 int store_i32_launch(int32_t* p, int32_t v, hipStream_t st) {
   hipLaunchKernelGGL(store_i32_kernel, dim3(1), dim3(64), 0, st, p, v);
+  Q35_HIP_TRY(hipGetLastError());
+  return Q35_OK;
+}
+
+int embed_seqs_launch(const int8_t* q, const float* s, int D, const int32_t* prompt, int ldp, const PfArg& sq, float* x,
+                      hipStream_t st) {
+  hipLaunchKernelGGL(embed_seqs_kernel, dim3(sq.rows), dim3(kPT), 0, st, q, s, D, prompt, ldp, sq, x);
+  Q35_HIP_TRY(hipGetLastError());
+  return Q35_OK;
+}
+
+int last_rows_launch(const float* x, int ldx, int D, const PfArg& sq, float* h, int32_t* pos, hipStream_t st) {
+  hipLaunchKernelGGL(last_rows_kernel, dim3(sq.n), dim3(kPT), 0, st, x, ldx, D, sq, h, pos);
   Q35_HIP_TRY(hipGetLastError());
   return Q35_OK;
 }
@@ -845,11 +884,11 @@ int gate_prompt_launch(const float* x, int ldx, int T, int K, const float* wb, c
 
 int gdn_prefill_launch(const GdnPrefill& a, hipStream_t st) {
   if (!a.raw || !a.conv_state || !a.conv_w || !a.bg || !a.scr || !a.S || !a.out) return fail(Q35_E_ARG, "gdn_prefill: null pointer");
-  if (a.T < 1 || a.nh < 1 || a.nchunk != (a.T + kC - 1) / kC) return fail(Q35_E_SHAPE, "gdn_prefill: bad T / chunks");
+  if (a.sq.n < 1 || (a.sq.n > 1 && !a.sq.tab) || a.nh < 1) return fail(Q35_E_SHAPE, "gdn_prefill: bad sequences or heads");
   if ((a.ld_out % 4) != 0) return fail(Q35_E_ALIGN, "gdn_prefill: output rows must be 16-byte aligned");
-  hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(a.nchunk * a.nh), dim3(kPP), 0, st, a);
+  hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(a.sq.chunks * a.nh), dim3(kPP), 0, st, a);
   Q35_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(gdn_chunk_state_kernel, dim3(kNsl * a.nh), dim3(kST), 0, st, a);
+  hipLaunchKernelGGL(gdn_chunk_state_kernel, dim3(kNsl * a.nh * a.sq.n), dim3(kST), 0, st, a);
   Q35_HIP_TRY(hipGetLastError());
   return Q35_OK;
 }
@@ -865,16 +904,16 @@ int gated_norm_rows_launch(const float* o, int ldo, const float* z, int ldz, con
 int attn_prefill_launch(const AttnPrefill& a, hipStream_t st) {
   if (!a.qg || !a.k || !a.v || !a.qnw || !a.knw || !a.rcos || !a.rsin || !a.kc || !a.vc || !a.qbuf || !a.out)
     return fail(Q35_E_ARG, "attention prefill: null pointer");
-  if (a.T < 1) return Q35_OK;
+  if (a.sq.n < 1) return Q35_OK;
   if (a.nkv < 1 || a.nh % a.nkv != 0 || kRows % (a.nh / a.nkv) != 0) return fail(Q35_E_SHAPE, "attention prefill: heads");
-  if (a.p0 < 0 || (int64_t)a.p0 + a.T > a.tmax) return fail(Q35_E_SHAPE, "attention prefill: positions past tmax");
+  // (a table's sequences are checked by the caller that builds it)
+  if (a.sq.n == 1 && (a.sq.one.p0 < 0 || (int64_t)a.sq.one.p0 + a.sq.one.T > a.tmax))
+    return fail(Q35_E_SHAPE, "attention prefill: positions past tmax");
   if (a.rot < 2 || a.rot > kHdP || (a.rot % 2) != 0) return fail(Q35_E_SHAPE, "attention prefill: rotary dims");
   if ((a.ld_qg % 4) != 0 || (a.ld_out % 4) != 0) return fail(Q35_E_ALIGN, "attention prefill: row alignment");
-  hipLaunchKernelGGL(attn_prefill_prep_kernel, dim3(a.T * (a.nh + a.nkv)), dim3(kPT), 0, st, a);
+  hipLaunchKernelGGL(attn_prefill_prep_kernel, dim3(a.sq.rows * (a.nh + a.nkv)), dim3(kPT), 0, st, a);
   Q35_HIP_TRY(hipGetLastError());
-  const int QT = kRows / (a.nh / a.nkv);
-  const int nqt = (a.T + QT - 1) / QT;
-  hipLaunchKernelGGL(attn_prefill_kernel, dim3(nqt * a.nkv), dim3(kAT), 0, st, a);
+  hipLaunchKernelGGL(attn_prefill_kernel, dim3(a.sq.tiles * a.nkv), dim3(kAT), 0, st, a);
   Q35_HIP_TRY(hipGetLastError());
   return Q35_OK;
 }

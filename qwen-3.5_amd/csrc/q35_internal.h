@@ -677,6 +677,58 @@ int mb_lm_head_launch(const int8_t* q, const float* sT, int32_t V, int32_t K, co
 int mb_scale_transpose_launch(const float* s, int32_t V, int32_t K, float* sT, hipStream_t st);
 
 // ------------------------------------------------------------------ prompt (seq_len > 1) path
+// The sequences whose rows one prompt pass carries, one after another: sequence s has rows
+// [row0[s], row0[s + 1]) at positions p0[s].. of state slot slot[s], chunks [chunk0[s], chunk0[s + 1])
+// of the chunked rule and attention query tiles from tile0[s].
+constexpr int kPfSeqs = 32;
+struct PfSeqs {
+  int32_t n = 0;
+  int32_t row0[kPfSeqs + 1] = {}, chunk0[kPfSeqs + 1] = {}, tile0[kPfSeqs + 1] = {};
+  int32_t p0[kPfSeqs] = {}, slot[kPfSeqs] = {};
+  void add(int32_t rows, int32_t pos, int32_t sl, int32_t chunk, int32_t tile) {
+    row0[n + 1] = row0[n] + rows;
+    chunk0[n + 1] = chunk0[n] + (rows + chunk - 1) / chunk;
+    tile0[n + 1] = tile0[n] + (rows + tile - 1) / tile;
+    p0[n] = pos;
+    slot[n] = sl;
+    ++n;
+  }
+};
+struct PfSeq { int32_t tb, T, p0, slot, cbeg, nchunk, tile0; };
+// How the kernels get them: one sequence in the arguments themselves (a table there, 670 bytes more,
+// cost each launch 0.3 us), more in a device copy of the table.
+struct PfArg {
+  int32_t n = 0, rows = 0, chunks = 0, tiles = 0;
+  PfSeq one{};
+  const PfSeqs* tab = nullptr;
+};
+inline PfArg pf_arg(const PfSeqs& q, const PfSeqs* tab) {
+  PfArg a;
+  a.n = q.n; a.rows = q.row0[q.n]; a.chunks = q.chunk0[q.n]; a.tiles = q.tile0[q.n];
+  if (q.n) a.one = PfSeq{0, q.row0[1], q.p0[0], q.slot[0], 0, q.chunk0[1], 0};
+  a.tab = tab;
+  return a;
+}
+Q35_DEV PfSeq pf_nth(const PfArg& a, int s) {
+  if (a.n == 1) return a.one;
+  const PfSeqs& q = *a.tab;
+  return PfSeq{q.row0[s], q.row0[s + 1] - q.row0[s], q.p0[s], q.slot[s], q.chunk0[s], q.chunk0[s + 1] - q.chunk0[s], q.tile0[s]};
+}
+// The sequence of row, chunk or tile i (FIRST: the table's member; i uniform over a block)
+template <int32_t (PfSeqs::*FIRST)[kPfSeqs + 1]>
+Q35_DEV PfSeq pf_seq(const PfArg& a, int i) {
+  int s = 0;
+  if (a.n > 1)
+    while (s + 1 < a.n && i >= (a.tab->*FIRST)[s + 1]) ++s;
+  return pf_nth(a, s);
+}
+// Tokens per query tile of the prompt attention (16 query rows of one kv head).
+inline int32_t pf_attn_tile(int32_t nh, int32_t nkv) { return 16 / (nh / nkv); }
+// x[t] = embedding of the prompt id at its sequence's position, prompt[slot * ldp + position]
+int embed_seqs_launch(const int8_t* q, const float* s, int D, const int32_t* prompt, int ldp, const PfArg& sq, float* x,
+                      hipStream_t st);
+// h[slot] = x[last row of the sequence], pos[slot] = its last position
+int last_rows_launch(const float* x, int ldx, int D, const PfArg& sq, float* h, int32_t* pos, hipStream_t st);
 // *p = v on the stream (a kernel, so it can sit in a captured graph)
 int store_i32_launch(int32_t* p, int32_t v, hipStream_t st);
 // y[m] = RMSNorm(x[m]) * (1 + w) for M rows of K
@@ -689,39 +741,42 @@ int rms_rows_launch(float* x, int ldx, int M, int K, const float* w, float eps, 
 // [beta | g] rows of a prompt (x [T][ldx], softplus identity branch when its input exceeds 20)
 int gate_prompt_launch(const float* x, int ldx, int T, int K, const float* wb, const float* wa, const float* alog,
                        const float* dtb, int nh, float* out, hipStream_t st);
-// Gated DeltaNet over a prompt of T tokens (dk = dv = 128): causal conv continuing conv_state,
-// chunked gated delta rule continuing S.  scr: nh * nchunk * kGdnScratchPerChunk floats.
+// Gated DeltaNet over the prompt rows of sq's sequences (dk = dv = 128): causal conv continuing
+// conv_state, chunked gated delta rule continuing S, each sequence's at its slot.  scr: nh * (all
+// chunks) * kGdnScratchPerChunk floats.
 constexpr int kGdnChunk = 64;
 constexpr int kGdnScratchPerChunk = 4 * 64 * 128 + 64 * 64 + 64;
 struct GdnPrefill {
   const float* raw = nullptr; int32_t ld_raw = 0;  // pre-conv q|k|v [T][conv_dim] (row stride ld_raw)
-  const float* conv_state = nullptr;               // [conv_dim][3] before the prompt
+  const float* conv_state = nullptr;               // [slot][conv_dim][3] before the prompt
   float* conv_state_out = nullptr;                 // written with the state after it (may alias)
   const float* conv_w = nullptr;                   // [conv_dim][4]
   const float* bg = nullptr; int32_t ld_bg = 0;    // [T][2 nh]: beta | g
   float* scr = nullptr;
-  float* S = nullptr;                              // [nh][128][128], updated
+  float* S = nullptr;                              // [slot][nh][128][128], updated
   float* out = nullptr; int32_t ld_out = 0;        // [T][nh*128] core output (before the gated norm)
-  int32_t T = 0, nh = 0, key_dim = 0, nchunk = 0;
+  int32_t nh = 0, key_dim = 0;
   float qscale = 0.f;
+  PfArg sq;
 };
 int gdn_prefill_launch(const GdnPrefill& a, hipStream_t st);
 // out[t][h*128 + i] = (w[i] * (o * rsqrt(mean(o^2) + eps))) * silu(z), per 128-wide head
 int gated_norm_rows_launch(const float* o, int ldo, const float* z, int ldz, const float* w, int T, int nh, float eps,
                            float* out, int ldout, hipStream_t st, float* amax = nullptr);
 // out[t][k] = gu[t][F + k] * silu(gu[t][k])
-// Attention over a prompt of T tokens at positions p0..p0+T-1 (head_dim 256, one sequence).
+// Attention over the prompt rows of sq's sequences at their positions (head_dim 256).
 constexpr int kHdP = 256;
 struct AttnPrefill {
   const float* qg = nullptr; int32_t ld_qg = 0;  // q_proj rows, per head [query | gate]
   const float* k = nullptr; const float* v = nullptr; int32_t ld_kv = 0;
   const float* qnw = nullptr; const float* knw = nullptr; float eps = 1e-6f;
   const float* rcos = nullptr; const float* rsin = nullptr; int32_t rot = 0;
-  float* kc = nullptr; float* vc = nullptr; int32_t tmax = 0;  // [nkv][tmax][256]
-  int32_t p0 = 0, T = 0, nh = 0, nkv = 0;
+  float* kc = nullptr; float* vc = nullptr; int32_t tmax = 0;  // [slot][nkv][tmax][256]
+  int32_t nh = 0, nkv = 0;
   float* qbuf = nullptr;                        // scratch [T][nh][256]
   float* out = nullptr; int32_t ld_out = 0;     // [T][nh*256]
   float scale = 0.0625f;
+  PfArg sq;
 };
 int attn_prefill_launch(const AttnPrefill& a, hipStream_t st);
 

@@ -1,0 +1,36 @@
+"""Prompts of a batch that share prompt passes: every row's ids equal a run of its own, where prompts
+of one token, of a chunk of 64, of 63 and 65, more prompts than one pass takes (32), and prompts longer
+than a pass (1024 tokens, then a rest that shares a pass with the next rows) meet; a second turn
+continues the rows' caches at different positions."""
+import numpy as np
+import pytest
+
+import q35
+
+pytestmark = pytest.mark.gpu
+
+
+def dims():
+    return q35.make_dims(hidden=512, ffn=1536, vocab=8192, n_layers=4, lin_heads=4, attn_heads=4, kv_heads=2)
+
+
+@pytest.mark.parametrize("lens", [[1, 64, 63, 65, 2, 3, 17], [5] * 40, [1100, 3, 70, 1025, 30]])
+def test_batch_prompts_share_passes(lens):
+    print(f"[batch prompts] {len(lens)} rows, longest {max(lens)}", flush=True)
+    d, n_new, second = dims(), 6, 9
+    rng = np.random.default_rng(len(lens))
+    prompts = [rng.integers(0, d.vocab, n).astype(np.int32) for n in lens]
+    turn2 = [rng.integers(0, d.vocab, second + r % 3).astype(np.int32) for r in range(len(lens))]
+    tmax = max(lens) + 2 * n_new + second + 8
+    m = q35.TextForCausalLM(d, seed=3, tmax=tmax)
+    bt = q35.BatchDecoder(m, len(lens), tmax)
+    toks, _ = bt.generate(prompts, n_new, prefill=True)
+    toks2, _ = bt.generate(turn2, n_new, prefill=True)
+    for r in range(len(lens)):
+        m.reset()
+        want, _ = m.generate(prompts[r], n_new, mode="persistent", prefill=True)
+        want2, _ = m.generate(turn2[r], n_new, mode="persistent", prefill=True)
+        np.testing.assert_array_equal(toks[r], want, err_msg=f"row {r}")
+        np.testing.assert_array_equal(toks2[r], want2, err_msg=f"row {r}, second turn")
+    bt.close()
+    m.close()
