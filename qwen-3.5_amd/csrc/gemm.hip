@@ -221,6 +221,26 @@ __global__ __launch_bounds__(kGT) void gemm_kernel(const GArgs a) {
     }
 }
 
+// (part_0 + part_1) + ... in split order, every split's load issued before the first add
+template <int KS>
+Q35_DEV f32x4 sum_ks(const float* p, int64_t stride) {
+  f32x4 v[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) v[s] = *(const Q35_GLOBAL f32x4*)(p + s * stride);
+#pragma unroll
+  for (int s = 1; s < KS; ++s) v[0] += v[s];
+  return v[0];
+}
+Q35_DEV f32x4 sum_ks(const float* p, int ks, int64_t stride) {
+  switch (ks) {  // (the launcher splits by powers of two)
+    case 1: return sum_ks<1>(p, stride);
+    case 2: return sum_ks<2>(p, stride);
+    case 4: return sum_ks<4>(p, stride);
+    case 8: return sum_ks<8>(p, stride);
+    default: return sum_ks<16>(p, stride);
+  }
+}
+
 // Split-K finish: y (+)= sum over the splits of part[s][m][c], in split order (deterministic);
 // one thread per 4 consecutive columns of one row.
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GArgs a) {
@@ -233,16 +253,42 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GArgs a) {
   for (int s = 1; s < kGemmMaxSeg; ++s)
     if (s < a.nseg && c >= a.seg[s].c0) sg = a.seg[s];
   const float* p = a.part + (int64_t)m * a.ncat + c;
-  float4 v = *(const float4*)p;
-  for (int s = 1; s < a.ksplit; ++s) {
-    const float4 u = *(const float4*)(p + (int64_t)s * a.M * a.ncat);
-    v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
-  }
+  f32x4 v = sum_ks(p, a.ksplit, (int64_t)a.M * a.ncat);
   float* y = sg.y + (int64_t)m * sg.ldy + (c - sg.c0);
   if (a.accumulate) {
-    v.x += y[0]; v.y += y[1]; v.z += y[2]; v.w += y[3];
+    v[0] += y[0]; v[1] += y[1]; v[2] += y[2]; v[3] += y[3];
   }
-  y[0] = v.x; y[1] = v.y; y[2] = v.z; y[3] = v.w;
+  y[0] = v[0]; y[1] = v[1]; y[2] = v[2]; y[3] = v[3];
+}
+
+// Split-K finish of gate | up (concatenated columns, N / 2 each) with the SwiGLU: act = up * silu(gate)
+// of the sums in split order, and each row's largest |act| raised in act_amax.  One thread per 4
+// columns, blocks of 1024 columns of one row.
+__global__ __launch_bounds__(256) void gemm_swiglu_reduce_kernel(const GArgs a) {
+  __shared__ float sh[4];
+  const int F = a.ncat >> 1, nb = (F + 1023) / 1024, m = blockIdx.x / nb;
+  const int j = (blockIdx.x % nb) * 1024 + 4 * threadIdx.x;
+  float mx = 0.f;
+  if (j < F) {
+    const float* p = a.part + (int64_t)m * a.ncat + j;
+    const int64_t st = (int64_t)a.M * a.ncat;
+    const f32x4 g = sum_ks(p, a.ksplit, st);
+    f32x4 u = sum_ks(p + F, a.ksplit, st);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      u[r] *= silu_f(g[r]);
+      mx = fmaxf(mx, fabsf(u[r]));
+    }
+    *(f32x4*)(a.act + (int64_t)m * a.ld_act + j) = u;
+  }
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) {  // (non-negative floats order as their bit patterns)
+    mx = fmaxf(fmaxf(sh[0], sh[1]), fmaxf(sh[2], sh[3]));
+    __hip_atomic_fetch_max((Q35_GLOBAL uint32_t*)(a.act_amax + m), __float_as_uint(mx), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // ------------------------------------------------------------------ f16 matrix cores (Q35_KN_MB)
@@ -447,7 +493,7 @@ __global__ __launch_bounds__(kGT, 2) void hgemm_kernel(const GArgs a) {
 
   // lane holds D[n = 16 nt + 4 g + r][m = 16 i + c] of the wave's tile: 4 consecutive columns of
   // one row per (nt, i)
-  if (a.act) {
+  if (a.act && a.nseg == 1) {
     // SwiGLU: the tile's column blocks are gate (wave wn = 0) and up (wn = 1) of the same 64 act
     // columns, at the same lane positions; the up wave hands its values over through LDS (the x
     // staging buffer, idle after the loop's last barrier)
@@ -495,7 +541,7 @@ __global__ __launch_bounds__(kGT, 2) void hgemm_kernel(const GArgs a) {
     for (int nt = 0; nt < 4; ++nt) {
       const int col = n0 + wn * 64 + 16 * nt + 4 * g;
       mf4 v = acc[nt][i] * inv;
-      if (a.ksplit > 1) {
+      if (a.ksplit > 1 || a.act) {
         *(mf4*)(a.part + ((int64_t)split * a.M + row) * a.ncat + sg.c0 + col) = v;
       } else {
         mf4* y = (mf4*)(sg.y + (int64_t)row * sg.ldy + col);
@@ -577,6 +623,11 @@ int launch_mb(const GemmCall& c, int ksplit, hipStream_t st) {
   if (prep_blocks > 0) hipLaunchKernelGGL(hgemm_prep_kernel, dim3((unsigned)prep_blocks), dim3(256), 0, st, a);
   hipLaunchKernelGGL((hgemm_kernel<BM>), dim3(a.nblocks), dim3(kGT), 0, st, a);
   Q35_HIP_TRY(hipGetLastError());
+  if (c.act && c.nseg == 2) {
+    hipLaunchKernelGGL(gemm_swiglu_reduce_kernel, dim3((unsigned)(c.M * ((ncat / 2 + 1023) / 1024))), dim3(256), 0, st, a);
+    Q35_HIP_TRY(hipGetLastError());
+    return Q35_OK;
+  }
   const bool defer = c.defer_reduce && c.nseg == 1;
   if (c.ksplit_out) *c.ksplit_out = defer ? ksplit : 1;  // partial sums the caller must add
   if (ksplit > 1 && !defer) {
@@ -604,13 +655,16 @@ void gemm_pick_mb(const GemmCall& c, int* bm, int* ksplit) {
   double best = 1e300;
   *bm = 64;
   *ksplit = 1;
-  if (c.act) return;  // (the SwiGLU epilogue needs whole sums)
-  for (int ks = 1; ks <= kGemmMaxSplit; ks *= 2) {
+  if (c.act && c.nseg == 1) return;  // (the SwiGLU epilogue needs whole sums)
+  for (int ks = 1; ks <= kGemmMaxSplitMb; ks *= 2) {
     if (ks > 1 && (!c.part || c.part_floats < (size_t)ks * c.M * ncat || c.K / kHBK < 2 * ks)) break;
+    // past 4 splits only while half of them would leave half the CUs idle: the splits' reading back
+    // then costs more than the model's rate (2048 x 6144, 64 rows: 8 splits 23.3 us, 4 splits 22.4)
+    if (ks > kGemmMaxSplit && tiles * (ks / 2) > cus / 2) break;
     const int steps = (c.K / kHBK + ks - 1) / ks;
     const long long per_cu = (tiles * ks + cus - 1) / cus;
     double cost = per_cu <= 1 ? steps * 1.09e-6 : (double)per_cu * steps * 0.91e-6;
-    if (ks > 1) cost += (double)c.M * ncat * (ks + 1) * 4.0 / 4e12 + 3e-6;
+    if (ks > 1) cost += (double)c.M * ncat * (ks + 1) * 4.0 / 4e12 + (c.defer_reduce ? 0.0 : 3e-6);
     if (cost < best * 0.97) { best = cost; *ksplit = ks; }
   }
 }
@@ -669,8 +723,9 @@ int gemm_launch(const GemmCall& c, hipStream_t st) {
           (reinterpret_cast<uintptr_t>(s.y) & 15) || (s.ldy % 4))
         return fail(Q35_E_ALIGN, "gemm: Q35_KN_MB needs 16-byte aligned q, scales and y rows");
     }
-    if (c.act && (c.nseg != 1 || !c.act_amax || (c.ld_act % 4) != 0 || (reinterpret_cast<uintptr_t>(c.act) & 15)))
-      return fail(Q35_E_ARG, "gemm: the SwiGLU output needs one segment, row maxima and 16-byte aligned rows");
+    if (c.act && (c.nseg > 2 || (c.nseg == 2 && (c.seg[0].N != c.seg[1].N || !c.part ||
+                                                 c.part_floats < (size_t)c.M * 2 * c.seg[0].N)) || !c.act_amax || (c.ld_act % 4) != 0 || (reinterpret_cast<uintptr_t>(c.act) & 15)))
+      return fail(Q35_E_ARG, "gemm: the SwiGLU output needs one segment (or gate, up and partials), row maxima and 16-byte aligned rows");
     int bm = 64, ks = 1;
     gemm_pick_mb(c, &bm, &ks);
     return launch_mb<64>(c, ks, st);

@@ -280,6 +280,9 @@ int persistent(q35_model* m, int n, hipStream_t st, const int32_t* stop_ids = nu
 
 // ---- prompt path (TextForCausalLM::forward at seq_len > 1, model.rs:27-84,130-138)
 constexpr int kPrefillCap = 1024;  // tokens per pass; longer prompts run in passes
+// Rows up to which gate | up splits K and applies the SwiGLU in a second kernel: the fused epilogue
+// needs whole sums, and one 64-row tile is 96 blocks of the 2B shape's 12288 columns
+constexpr int kPrefillSplitGu = 64;
 
 SeqView model_view(q35_model* m) {
   SeqView v;
@@ -453,6 +456,11 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
     GemmCall g;
     g.x = m->pf_xn; g.ldx = H; g.M = T; g.K = H; g.nseg = 1;
     g.seg[0] = GemmSeg{W.gu.q, W.gu.s, m->pf_y, 2 * F, Q35_KN_MB, LDY, W.gu.smax};
+    if (T <= kPrefillSplitGu) {
+      g.nseg = 2;
+      g.seg[0] = seg(L.gate, W.gate, m->pf_y, LDY);
+      g.seg[1] = seg(L.up, W.up, m->pf_y + F, LDY);
+    }
     g.part = m->pf_part; g.part_floats = gemm_part_floats(m->pf_cap, d.hidden); g.aux = m->pf_aux; g.amax = m->pf_aux;
     g.act = m->pf_a; g.ld_act = F; g.act_amax = m->pf_act_max;
     if ((rc = gemm_launch(g, st))) return rc;

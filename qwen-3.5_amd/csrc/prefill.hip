@@ -63,6 +63,16 @@ Q35_DEV void block_max256_store(float v, float* sh, float* dst) {
 // kRmsHeld * 4 * 256 floats (K a multiple of 4, rows 16-byte aligned) stay in registers between
 // the sum of squares and the scaling (one read of x); longer ones are read twice.
 constexpr int kRmsHeld = 4;  // float4 per thread held
+// (part_0 + part_1) + ... , every split's load issued before the first add
+template <int N>
+Q35_DEV float4 sum_parts(const float* p, int64_t stride) {
+  q35_f32x4 v[N];
+#pragma unroll
+  for (int s = 0; s < N; ++s) v[s] = *(const Q35_GLOBAL q35_f32x4*)(p + s * stride);
+#pragma unroll
+  for (int s = 1; s < N; ++s) v[0] += v[s];
+  return make_float4(v[0][0], v[0][1], v[0][2], v[0][3]);
+}
 __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K, const float* w, float eps,
                                                        float* y, int ldy, float* amax, const float* part,
                                                        int nsplit, int64_t sstride, int ldp, float* clear) {
@@ -88,10 +98,18 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
       for (int u = 0; u < kRmsHeld; ++u) {
         const int k = 4 * (threadIdx.x + u * kPT);
         if (k < K) {
-          float4 t = *(const float4*)(pr + k);
-          for (int s = 1; s < nsplit; ++s) {
-            const float4 q = *(const float4*)(pr + s * sstride + k);
-            t.x += q.x; t.y += q.y; t.z += q.z; t.w += q.w;
+          float4 t;
+          switch (nsplit) {
+            case 2: t = sum_parts<2>(pr + k, sstride); break;
+            case 4: t = sum_parts<4>(pr + k, sstride); break;
+            case 8: t = sum_parts<8>(pr + k, sstride); break;
+            case 16: t = sum_parts<16>(pr + k, sstride); break;
+            default:
+              t = *(const float4*)(pr + k);
+              for (int s = 1; s < nsplit; ++s) {
+                const float4 q = *(const float4*)(pr + s * sstride + k);
+                t.x += q.x; t.y += q.y; t.z += q.z; t.w += q.w;
+              }
           }
           v[u] = make_float4(t.x + v[u].x, t.y + v[u].y, t.z + v[u].z, t.w + v[u].w);
           *(float4*)(xr + k) = v[u];

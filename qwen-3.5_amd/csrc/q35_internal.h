@@ -502,7 +502,8 @@ struct GemmCall {
   // Q35_KN_MB, one segment whose 64-column blocks alternate gate and up (block 2 j: gate columns
   // 64 j .., block 2 j + 1: up columns 64 j ..): the launch writes act[m][64 j + c] =
   // up * silu(gate) (N / 2 columns) instead of y, and raises act_amax[m] (zero beforehand) to each
-  // row's max |act|; K is not split
+  // row's max |act|; K is not split.  With two segments (gate, up; each N columns) and partials, K may
+  // be split and a second kernel forms the same rows.
   float* act = nullptr;
   int32_t ld_act = 0;
   float* act_amax = nullptr;
@@ -513,8 +514,12 @@ int gemm_launch(const GemmCall& c, hipStream_t st);
 // Tile shape and K splits the launcher picks for c (BM x BN, ksplit).
 int gemm_pick(const GemmCall& c, int* bm, int* bn, int* ksplit);
 // Partial floats that let gemm_launch consider up to kGemmMaxSplit K splits for M rows of N columns.
-constexpr int kGemmMaxSplit = 4;
-inline size_t gemm_part_floats(int M, int64_t N) { return (size_t)kGemmMaxSplit * M * N; }
+// Few rows make few tiles, so the MB launches split further: one 64-row tile of a 2048-wide projection
+// is 16 blocks for 256 CUs.
+constexpr int kGemmMaxSplit = 4, kGemmMaxSplitMb = 16;
+inline size_t gemm_part_floats(int M, int64_t N) {
+  return (size_t)(M <= 64 ? 16 : (M <= 128 ? 8 : kGemmMaxSplit)) * M * N;
+}
 
 // ------------------------------------------------------------------ Q8F NK matvec / lm_head
 struct NkCall {
