@@ -82,9 +82,9 @@ size_t acc_bytes(const q35_dims& d, int B) {
 // ---- the multi-row path of the layer calls and q8_gemv (mvm.hip), unless a buffer's alignment or
 // a shape asks for the one-row kernel's row groups.  Layer calls take it from 2 rows on (device time
 // of the 2B MLP at 2 rows 27.9 -> 24.0 us from KN weights, 27.3 -> 20.8 tiled; attention 30.0 -> 25.9,
-// DeltaNet 28.2 -> 21.7); q8_gemv from 4 rows, where the one launch of the one-row kernel takes as
-// long as the two launches' host time (2048 x 6144 at 4 rows: 14.0 -> 9.4 us on the device, 14.45
-// issued one by one either way; at 2 rows 12.9 against 14.7 issued one by one).
+// DeltaNet 28.2 -> 21.7); q8_gemv from 4 rows: below, the second launch's host time is more than the
+// kernel saves (2048 x 6144 at 4 rows: 14.0 -> 9.4 us on the device; 2048 x 512 issued one by one: at
+// 3 rows 8.5 us with the one launch, at 5 rows 18.6 -> 10.2 with the two).
 constexpr int kMvmMin = 2, kMvmGemvMin = 4;
 MvmSeg mvm_seg(const q35_q8f& W) { return MvmSeg{W.q, W.scale, W.cols, W.layout == Q35_KN_TILED ? 1 : 0}; }
 

@@ -10,6 +10,7 @@ squeezes [1,1,K] and panics otherwise) and q8_gemv_partial_sum sums every input 
 reference kernel skips rows when K / splits is not a multiple of 8, kernels.rs:119-133,504).
 """
 import atexit
+import functools
 
 import numpy as np
 import torch
@@ -29,7 +30,9 @@ atexit.register(release_workspaces)
 
 
 def _stream():
-    return ctypes_stream(torch.cuda.current_stream())
+    # the current stream's handle without building a torch.cuda.Stream around it (1.5 us of the 12.6
+    # that a small call took on the host)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def ctypes_stream(s):
@@ -41,7 +44,8 @@ def workspace(nbytes, device=None, key="default"):
     its completion counters and fixed-point accumulators zero again, so a buffer serves every
     later call of the same entry point in stream order; different entry points lay out their
     workspace differently and get separate buffers (`key`)."""
-    device = torch.device(device or "cuda")
+    if type(device) is not torch.device:
+        device = torch.device(device or "cuda")
     k = (key, device.type, device.index if device.index is not None else torch.cuda.current_device())
     buf = _workspaces.get(k)
     if buf is None or buf.numel() < nbytes:
@@ -132,31 +136,35 @@ class Q8FTensor:
 
 
 def _rows(x, k):
-    x2 = x.reshape(-1, k)
+    x2 = x if x.dim() == 2 and x.shape[1] == k else x.reshape(-1, k)
     assert x2.dtype == torch.float32
     return x2.contiguous()
 
 
+@functools.lru_cache(maxsize=1024)
+def _gemv_ws_bytes(M, rows, cols, layout):
+    """q35_q8_gemv_ws_bytes, a function of the row count, the shape and the layout alone."""
+    return L.lib().q35_q8_gemv_ws_bytes(M, L.Q8F(None, None, rows, cols, layout))
+
+
+def _gemv(fn, hidden_states, weights):
+    x = _rows(hidden_states, weights.in_dim)
+    M, N = x.shape[0], weights.out_dim
+    y = x.new_empty((M, N))
+    ws = workspace(_gemv_ws_bytes(M, weights.rows, weights.cols, weights.layout), x.device, "gemv")
+    rc = fn(x.data_ptr(), M, weights.desc(), y.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
+    if rc:
+        L.check(rc)
+    return y if hidden_states.dim() == 2 else y.reshape(*hidden_states.shape[:-1], N)
+
+
 def q8_gemv(hidden_states, weights: Q8FTensor):
     """y = hidden_states @ dequant(W); hidden_states [..., K] -> [..., N]."""
-    K, N = weights.in_dim, weights.out_dim
-    x = _rows(hidden_states, K)
-    y = torch.empty((x.shape[0], N), dtype=torch.float32, device=x.device)
-    W = weights.desc()
-    ws = workspace(L.lib().q35_q8_gemv_ws_bytes(x.shape[0], W), x.device, "gemv")
-    L.check(L.lib().q35_q8_gemv(x.data_ptr(), x.shape[0], W, y.data_ptr(), ws.data_ptr(), ws.numel(), _stream()))
-    return y.reshape(*hidden_states.shape[:-1], N)
+    return _gemv(L.lib().q35_q8_gemv, hidden_states, weights)
 
 
 def q8_gemv_partial_sum(hidden_states, weights: Q8FTensor):
-    K, N = weights.in_dim, weights.out_dim
-    x = _rows(hidden_states, K)
-    y = torch.empty((x.shape[0], N), dtype=torch.float32, device=x.device)
-    W = weights.desc()
-    ws = workspace(L.lib().q35_q8_gemv_ws_bytes(x.shape[0], W), x.device, "gemv")
-    L.check(L.lib().q35_q8_gemv_partial_sum(x.data_ptr(), x.shape[0], W, y.data_ptr(), ws.data_ptr(), ws.numel(),
-                                            _stream()))
-    return y.reshape(*hidden_states.shape[:-1], N)
+    return _gemv(L.lib().q35_q8_gemv_partial_sum, hidden_states, weights)
 
 
 def q8_lm_head(hidden_states, embeddings: Q8FTensor):
@@ -164,7 +172,7 @@ def q8_lm_head(hidden_states, embeddings: Q8FTensor):
     assert embeddings.layout == L.Q35_NK
     V, D = embeddings.q.shape
     x = _rows(hidden_states, D)
-    y = torch.empty((x.shape[0], V), dtype=torch.float32, device=x.device)
+    y = x.new_empty((x.shape[0], V))
     L.check(L.lib().q35_q8_lm_head(x.data_ptr(), x.shape[0], embeddings.desc(), y.data_ptr(), _stream()))
     return y.reshape(*hidden_states.shape[:-1], V)
 
