@@ -5,13 +5,15 @@
 //
 // Split-T ("flash decoding") in two kernels:
 //  * chunk kernel, block (b, kv head g, chunk c) over `chunk` cached tokens for the rep = nh/nkv
-//    query heads of g, so each K/V row is read once for all of them.  Wave w takes tokens
-//    w, w+4, ...; a lane owns 4 of the 256 dims (one float4 of every row, 1 KB per wave per row).
-//    Every K and V row of a batch of 2 tokens per wave is requested before the first is used,
-//    and the next batch's rows before the current batch is computed, so a chunk costs one memory
-//    round trip rather than one per token.  Scores feed an online softmax (running max, sum and
-//    P.V per head in registers); the 4 waves are combined through LDS.  A block whose chunk is
-//    the only one writes the gated output; otherwise it publishes (max, sum, o[rep][256]).
+//    query heads of g, so each K/V row is read once for all of them.  Wave w takes 4 tokens of every
+//    16, one per 16-lane row; lane j of a row owns dims 4 j + 64 i (i < 4) of its token, so a score is
+//    16 multiply-adds and 4 row rotations for 4 tokens at once (with a whole wave on one token the
+//    64-lane sums were most of the kernel's vector work).  The next 4 tokens' rows are requested
+//    before the current ones are computed.  Each 16-lane row keeps its own online softmax (running
+//    max, sum and P.V per head in registers); rows and waves are combined at the end.  A block whose
+//    chunk is the only one writes the gated output; otherwise it publishes (max, sum, o[rep][256]).
+//    Bound: the K/V stream.  16 rows over 8192-token caches at mixed positions (335 MB, both kernels):
+//    91.2 -> 63.0 us, 5.3 TB/s.
 //  * merge kernel, block (b, query head h, 64-dim slice): chunk weights 2^(m_c - M) in LDS (the
 //    maxima are kept in log2 units), 4 threads per dim each summing a quarter of the chunks (16
 //    loads in flight), then the gate.
@@ -29,12 +31,10 @@ constexpr int kNW = kThreads / 64;
 constexpr int kHd = 256;
 constexpr int kMaxRep = 4;
 constexpr int kMinChunk = 16;
-constexpr int kMaxChunk = 256;     // tokens per block
+constexpr int kMaxChunk = 512;     // tokens per block
 constexpr int kMaxChunks = 1024;   // chunks per (b, kv head): the merge keeps their weights in LDS
-#ifndef Q35_ATT_BATCH
-#define Q35_ATT_BATCH 2
-#endif
-constexpr int kBatch = Q35_ATT_BATCH;  // tokens per wave per load batch
+constexpr int kMaxTokens = 262144; // longest cache
+constexpr int kStep = 4 * kNW;         // tokens per block iteration
 
 struct AttnArgs {
   AttnCall c;
@@ -55,12 +55,23 @@ Q35_DEV float4 ldf4(const float* p) {
   return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
 }
 
+// a summed over lanes l and l ^ 32 in the lower half, b in the upper half (v_permlane32_swap)
+Q35_DEV float add_swap32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// a summed over lanes l and l ^ 16 in even 16-lane rows, b in odd rows (v_permlane16_swap)
+Q35_DEV float add_swap16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 Q35_DEV bool pos_ok(const AttnArgs& A, int b, int* pos) {
   *pos = A.c.pos[b];
   return *pos >= 0 && *pos < A.c.tmax;
 }
 
-__global__ __launch_bounds__(kThreads) void attn_chunk_kernel(const AttnArgs A) {
+__global__ __launch_bounds__(kThreads, 2) void attn_chunk_kernel(const AttnArgs A) {
   const AttnCall& a = A.c;
   __shared__ __align__(16) float qn[kMaxRep][kHd];
   __shared__ __align__(16) float kn[kHd];
@@ -88,21 +99,22 @@ __global__ __launch_bounds__(kThreads) void attn_chunk_kernel(const AttnArgs A) 
   const size_t cache_off = (((size_t)b * a.nkv + g) * a.tmax) * kHd;
   const float* Kc = a.kc + cache_off;
   const float* Vc = a.vc + cache_off;
-  // rows of wave wid: t0 + wid + 4 i, i < nw_tok; rows at or past pos (the new token) are not read
-  const int nw_tok = (len - wid + kNW - 1) / kNW;
-  // two register buffers of kBatch rows each (fixed indices: the batch loop below is unrolled by 2)
-  float4 k0b[kBatch], v0b[kBatch], k1b[kBatch], v1b[kBatch];
-  auto load_batch = [&](int bi, float4 (&kb)[kBatch], float4 (&vb)[kBatch]) {
+  // iteration it: the lane's token t0 + 16 it + 4 wid + tg; tokens at or past pos (the new one) are
+  // not read (rows clamped into the cache, masked when used).  Two register buffers, so the
+  // iteration loop is unrolled by two.
+  const int j = lane & 15, tg = lane >> 4;
+  const int nit = (len + kStep - 1) / kStep;
+  q35_f32x4 k0b[4], v0b[4], k1b[4], v1b[4];
+  auto load_it = [&](int it, q35_f32x4 (&kb)[4], q35_f32x4 (&vb)[4]) {
+    const int t = max(0, min(t0 + kStep * it + 4 * wid + tg, pos - 1));
+    const float* kr = Kc + (size_t)t * kHd + 4 * j;
+    const float* vr = Vc + (size_t)t * kHd + 4 * j;
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int t = t0 + wid + kNW * (bi * kBatch + u);
-      const int tr = max(0, min(t, pos - 1));  // clamped into the cache; masked when used
-      kb[u] = ldf4(Kc + (size_t)tr * kHd + 4 * lane);
-      vb[u] = ldf4(Vc + (size_t)tr * kHd + 4 * lane);
-    }
+    for (int i = 0; i < 4; ++i) kb[i] = __builtin_nontemporal_load((const Q35_GLOBAL q35_f32x4*)(kr + 64 * i));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) vb[i] = __builtin_nontemporal_load((const Q35_GLOBAL q35_f32x4*)(vr + 64 * i));
   };
-  const int nbatch = (nw_tok + kBatch - 1) / kBatch;
-  if (nbatch > 0) load_batch(0, k0b, v0b);
+  load_it(0, k0b, v0b);
 
   // q heads (wave w -> head g*rep + w), plus k/v of the new token in the chunk holding it
   for (int w = wid; w < rep + (has_new ? 2 : 0); w += kNW) {
@@ -150,73 +162,98 @@ __global__ __launch_bounds__(kThreads) void attn_chunk_kernel(const AttnArgs A) 
     a.vc[cache_off + (size_t)pos * kHd + tid] = vn[tid];
   }
 
-  float q4[kMaxRep][4];
+  q35_f32x4 q4[kMaxRep][4];
 #pragma unroll
   for (int h = 0; h < kMaxRep; ++h)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) q4[h][i] = (h < rep) ? qn[h][4 * lane + i] : 0.f;
-  const float4 kn4 = *reinterpret_cast<const float4*>(&kn[4 * lane]);
-  const float4 vn4 = *reinterpret_cast<const float4*>(&vn[4 * lane]);
-  // online softmax per head: running max m, sum l, and acc = sum p v (this lane's 4 dims)
-  float m[kMaxRep], l[kMaxRep], acc[kMaxRep][4];
+    for (int i = 0; i < 4; ++i) q4[h][i] = *(const q35_f32x4*)&qn[min(h, rep - 1)][4 * j + 64 * i];
+  // online softmax per head and 16-lane row: running max m, sum l, and acc = sum p v (the lane's dims)
+  float m[kMaxRep], l[kMaxRep];
+  q35_f32x4 acc[kMaxRep][4];
 #pragma unroll
   for (int h = 0; h < kMaxRep; ++h) {
     m[h] = -INFINITY;
     l[h] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[h][i] = 0.f;
+    for (int i = 0; i < 4; ++i) acc[h][i] = q35_f32x4{0.f, 0.f, 0.f, 0.f};
   }
   // Scores are kept in log2 units (scale * log2 e folded in) so that every exponential is one
-  // hardware exp2; the running max is updated once per batch of kBatch tokens.
+  // hardware exp2; a head's sums are rescaled only when a token of the wave raises a maximum.
   const float sl2 = A.scale * 1.44269504088896341f;
-  auto compute = [&](int bi, const float4 (&kb)[kBatch], const float4 (&vb)[kBatch]) {
-    const int nb = min(kBatch, nw_tok - bi * kBatch);  // tokens of this batch (uniform in the wave)
+  auto compute = [&](int it, q35_f32x4 (&kb)[4], q35_f32x4 (&vb)[4]) {
+    const int t = t0 + kStep * it + 4 * wid + tg;
+    if (has_new && kStep * it + 4 * wid + 4 > pos - t0) {  // (uniform) the new token may be among these
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const q35_f32x4 kx = *(const q35_f32x4*)&kn[4 * j + 64 * i], vx = *(const q35_f32x4*)&vn[4 * j + 64 * i];
+        kb[i] = t == pos ? kx : kb[i];
+        vb[i] = t == pos ? vx : vb[i];
+      }
+    }
+    const bool in = t < t0 + len;
 #pragma unroll
     for (int h = 0; h < kMaxRep; ++h) {
       if (h >= rep) break;
-      float s[kBatch];
-      float bm = -INFINITY;
+      q35_f32x4 d = q4[h][0] * kb[0];
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int t = t0 + wid + kNW * (bi * kBatch + u);
-        const float4 kv = (t == pos) ? kn4 : kb[u];
-        s[u] = (u < nb) ? wave_sum(q4[h][0] * kv.x + q4[h][1] * kv.y + q4[h][2] * kv.z + q4[h][3] * kv.w) * sl2
-                        : -INFINITY;
-        bm = fmaxf(bm, s[u]);
+      for (int i = 1; i < 4; ++i) d += q4[h][i] * kb[i];
+      float s = (d[0] + d[1]) + (d[2] + d[3]);
+      s += row_ror<8>(s);
+      s += row_ror<4>(s);
+      s += row_ror<2>(s);
+      s += row_ror<1>(s);
+      s = in ? s * sl2 : -INFINITY;
+      const float mn = fmaxf(m[h], s);
+      if (__ballot(mn > m[h])) {
+        const float al = m[h] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[h] - mn);
+        l[h] *= al;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[h][i] *= al;
+        m[h] = mn;
       }
-      const float mn = fmaxf(m[h], bm);
-      const float al = __builtin_amdgcn_exp2f(m[h] - mn);  // 0 while m is -inf
-      l[h] *= al;
+      const float p = s == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s - mn);
+      l[h] += p;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[h][e] *= al;
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int t = t0 + wid + kNW * (bi * kBatch + u);
-        const float4 vv = (t == pos) ? vn4 : vb[u];
-        const float p = __builtin_amdgcn_exp2f(s[u] - mn);  // 0 for the masked slots
-        l[h] += p;
-        acc[h][0] += p * vv.x;
-        acc[h][1] += p * vv.y;
-        acc[h][2] += p * vv.z;
-        acc[h][3] += p * vv.w;
-      }
-      m[h] = mn;
+      for (int i = 0; i < 4; ++i) acc[h][i] += p * vb[i];
     }
   };
-  // the next batch's rows are requested before the current batch is computed
-  for (int bi = 0; bi < nbatch; bi += 2) {
-    if (bi + 1 < nbatch) load_batch(bi + 1, k1b, v1b);
-    compute(bi, k0b, v0b);
-    if (bi + 1 >= nbatch) break;
-    if (bi + 2 < nbatch) load_batch(bi + 2, k0b, v0b);
-    compute(bi + 1, k1b, v1b);
+  // the next iteration's rows are requested before the current ones are computed
+  for (int it = 0; it < nit; it += 2) {
+    if (it + 1 < nit) load_it(it + 1, k1b, v1b);
+    compute(it, k0b, v0b);
+    if (it + 1 >= nit) break;
+    if (it + 2 < nit) load_it(it + 2, k0b, v0b);
+    compute(it + 1, k1b, v1b);
   }
-  // combine the 4 waves (a wave with no token has m = -inf, weight 0)
+  // the wave's 4 rows: a common maximum, then the lane swaps add the rows and leave row tg with head
+  // tg (swap by 32 lanes pairs heads h and h + 2, by 16 lanes heads 0 and 1 of what is left)
+  float mw[kMaxRep], lw[kMaxRep];
 #pragma unroll
   for (int h = 0; h < kMaxRep; ++h) {
-    if (h >= rep) break;
-    *reinterpret_cast<float4*>(&wo[wid][h][4 * lane]) = make_float4(acc[h][0], acc[h][1], acc[h][2], acc[h][3]);
-    if (lane == 0) { wm[wid][h] = m[h]; wl[wid][h] = l[h]; }
+    float M = fmaxf(m[h], __shfl_xor(m[h], 16));
+    M = fmaxf(M, __shfl_xor(M, 32));
+    const float f = m[h] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[h] - M);
+    float L = l[h] * f;
+    L += __shfl_xor(L, 16);
+    L += __shfl_xor(L, 32);
+    mw[h] = M;
+    lw[h] = L;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[h][i] *= f;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    q35_f32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x0 = add_swap32(acc[0][i][e], acc[2][i][e]), x1 = add_swap32(acc[1][i][e], acc[3][i][e]);
+      r[e] = add_swap16(x0, x1);
+    }
+    *(q35_f32x4*)&wo[wid][tg][4 * j + 64 * i] = r;
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int h = 0; h < kMaxRep; ++h) { wm[wid][h] = mw[h]; wl[wid][h] = lw[h]; }
   }
   __syncthreads();
   const int grpi = b * a.nkv + g;
@@ -307,7 +344,9 @@ __global__ __launch_bounds__(kThreads) void attn_merge_kernel(const AttnArgs A) 
   }
 }
 
-// Tokens per chunk: about 512 chunk blocks over the (b, kv head, tmax) work, 16 .. 256 tokens.
+// Tokens per chunk: about 512 chunk blocks over the (b, kv head, tmax) work, 16 .. 512 tokens: two
+// blocks fit a CU, and a block's start (norms, rotary, first rows) is paid once per chunk (the 335 MB
+// case above with at most 64 / 128 / 256 / 512 tokens: 86 / 78 / 70.5 / 63 us).
 int pick_chunk(int32_t B, int32_t nkv, int32_t tmax) {
   const long long work = (long long)B * nkv * tmax;
   long long ch = (work + 511) / 512;
@@ -357,7 +396,7 @@ int attn_launch_split(const AttnCall& c, uint32_t* counters, char* scratch, size
   if ((size_t)c.B * c.nkv * c.tmax * c.hd > (size_t)1 << 40) return fail(Q35_E_SHAPE, "attention: cache too large");
   AttnLayout L = attn_layout(c.B, c.nkv, c.hd, c.tmax);
   if (!counters || !scratch || scratch_bytes < L.ml_bytes + L.o_bytes) return fail(Q35_E_WS, "attention: workspace too small");
-  if (L.nchunk > kMaxChunks) return fail(Q35_E_SHAPE, "attention: tmax too large for one merge");
+  if (c.tmax > kMaxTokens || L.nchunk > kMaxChunks) return fail(Q35_E_SHAPE, "attention: tmax too large for one merge");
   AttnArgs A;
   A.c = c;
   A.scale = (float)(1.0 / sqrt((double)c.hd));
