@@ -50,10 +50,6 @@ Q35_DEV float4 ld4(const float* f, const fx_t* x, size_t i) {
   return *reinterpret_cast<const float4*>(f + i);
 }
 Q35_DEV float ld1(const float* f, const fx_t* x, size_t i) { return x ? from_fx(x[i]) : f[i]; }
-Q35_DEV float4 ldf4(const float* p) {
-  const uint4 u = ldg16(p);
-  return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
-}
 
 // a summed over lanes l and l ^ 32 in the lower half, b in the upper half (v_permlane32_swap)
 Q35_DEV float add_swap32(float a, float b) {

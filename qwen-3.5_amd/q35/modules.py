@@ -18,6 +18,12 @@ def _p(t):
     return t.contiguous().data_ptr()
 
 
+def _sizes(d):
+    """The dims as a workspace key: a layer's workspace serves calls of the same sizes only (what one
+    size leaves in its split-K partials would lie in another's accumulators)."""
+    return bytes(memoryview(d))
+
+
 class GatedDeltaNet:
     def __init__(self, dims, in_proj_qkv: Q8FTensor, in_proj_z: Q8FTensor, out_proj: Q8FTensor, in_proj_b, in_proj_a,
                  a_log, dt_bias, conv_w, norm_w):
@@ -36,7 +42,7 @@ class GatedDeltaNet:
         x = hidden_states.reshape(-1, d.hidden).contiguous()
         B = x.shape[0]
         out = torch.empty_like(x)
-        ws = workspace(L.lib().q35_layer_ws_bytes(ctypes.byref(d), B, 1), x.device, ("gated_deltanet", B))
+        ws = workspace(L.lib().q35_layer_ws_bytes(ctypes.byref(d), B, 1), x.device, ("gated_deltanet", B, _sizes(d)))
         L.check(L.lib().q35_gated_deltanet_decode(ctypes.byref(d), ctypes.byref(self.w), x.data_ptr(), B,
                                                   conv_state.data_ptr(), recurrent_state.data_ptr(), out.data_ptr(),
                                                   ws.data_ptr(), ws.numel(), _stream()))
@@ -60,7 +66,7 @@ class Attention:
         B = x.shape[0]
         tmax = k_cache.shape[2]
         out = torch.empty_like(x)
-        ws = workspace(L.lib().q35_layer_ws_bytes(ctypes.byref(d), B, tmax), x.device, ("attention", B, tmax))
+        ws = workspace(L.lib().q35_layer_ws_bytes(ctypes.byref(d), B, tmax), x.device, ("attention", B, tmax, _sizes(d)))
         L.check(L.lib().q35_attention_decode(ctypes.byref(d), ctypes.byref(self.w), x.data_ptr(), B, k_cache.data_ptr(),
                                              v_cache.data_ptr(), tmax, pos.data_ptr(), rope_cos.data_ptr(),
                                              rope_sin.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), _stream()))
@@ -81,7 +87,7 @@ class MLP:
         x2 = x.reshape(-1, d.hidden).contiguous()
         B = x2.shape[0]
         out = torch.empty_like(x2)
-        ws = workspace(L.lib().q35_layer_ws_bytes(ctypes.byref(d), B, 1), x2.device, ("mlp", B))
+        ws = workspace(L.lib().q35_layer_ws_bytes(ctypes.byref(d), B, 1), x2.device, ("mlp", B, _sizes(d)))
         L.check(L.lib().q35_mlp_decode(ctypes.byref(d), ctypes.byref(self.w), x2.data_ptr(), B, out.data_ptr(),
                                        ws.data_ptr(), ws.numel(), _stream()))
         if check:

@@ -86,3 +86,27 @@ def test_layers_in_row_groups(B):
         one = host(att.forward(x[b:b + 1], k1, v1, dev(pos[b:b + 1]), dev(cs), dev(sn)))
         assert rel_l2(out_a[b], one[0]) <= 3e-6, b
         assert rel_l2(host(kd[b]), host(k1[0])) <= 2e-6 and rel_l2(host(vd[b]), host(v1[0])) <= 2e-6
+
+
+@pytest.mark.parametrize("hidden,ffn,heads", [(512, 1536, 4), (64, 64, 2), (2048, 6144, 16)])
+def test_one_row_layers_between_batches(hidden, ffn, heads):
+    """One-row MLP and DeltaNet calls equal the same row in a batch of three, call after call, whatever
+    sizes other layers of the process have (each size has a workspace of its own)."""
+    d = q35.make_dims(hidden=hidden, ffn=ffn, lin_heads=heads)
+    vd, cd = heads * 128, 3 * heads * 128
+    mlp = q35.MLP(d, *(q8_dev(q8(460 + i, *s), q35.Q35_KN) for i, s in
+                       enumerate([(hidden, ffn), (hidden, ffn), (ffn, hidden)])))
+    gdn = q35.GatedDeltaNet(d, *(q8_dev(q8(464 + i, *s), q35.Q35_KN).tiled() for i, s in
+                                 enumerate([(hidden, cd), (hidden, vd), (vd, hidden)])),
+                            dev(normal(468, (hidden, heads), 0.02)), dev(normal(469, (hidden, heads), 0.02)),
+                            dev(normal(470, (heads,), 0.5)), dev(np.ones(heads, np.float32)),
+                            dev(normal(471, (cd, 4), 0.5)), dev(1 + normal(472, (128,), 0.1)))
+    x = dev(normal(473, (3, hidden)))
+    cs, S = normal(474, (3, cd, 3)), normal(475, (3, heads, 128, 128), 0.1)
+    cs3, S3 = dev(cs), dev(S)
+    out_m, out_g = host(mlp.forward(x)), host(gdn.forward(x, cs3, S3))
+    for r in (0, 2, 1):
+        assert rel_l2(host(mlp.forward(x[r:r + 1], check=True))[0], out_m[r]) <= 3e-6, r
+        cs1, S1 = dev(cs[r:r + 1]), dev(S[r:r + 1])
+        assert rel_l2(host(gdn.forward(x[r:r + 1], cs1, S1))[0], out_g[r]) <= 3e-6, r
+        assert rel_l2(host(S1)[0], host(S3)[r]) <= 3e-6 and rel_l2(host(cs1)[0], host(cs3)[r]) <= 3e-6, r
