@@ -704,70 +704,91 @@ __global__ __launch_bounds__(kPT) void attn_prefill_prep_kernel(const AttnPrefil
 // prompt gives 128 x kv_heads blocks.  Its 4 waves take every 4th 16-key tile, each with its own
 // online softmax (f32, log2 units), and merge their (max, sum, output) in wave order at the end.
 // A wave computes S^T = K Q^T for its tile (lane l = 16 g + c16: keys 4 g + r of query row c16)
-// and O^T += V^T P^T, whose lane holds dims 16 i + 4 g + r of the same row c16: the row's running
-// max, sum and rescale stay in the lane (the 16 keys of a row sit in lanes c16 + 16 g, reduced by
-// two exchanges).  Keys and values pass through a per-wave LDS slot, the next tile's loaded into
-// registers while the current one is computed; the block's 16 query rows sit in LDS.
+// and O^T += V^T P^T: the row's running max, sum and rescale stay in the lane (the 16 keys of a row
+// sit in lanes c16 + 16 g, reduced by two exchanges).  Keys and values go from the cache straight
+// into the operand registers (as operand of product i, dim 64 (i / 4) + 4 c16 + i % 4 of a value row
+// makes every load 256 contiguous bytes of 4 rows): the next tile's keys are requested when the
+// current ones have been multiplied, its values after the current ones, so each load has half a
+// tile's products to land, and without staging two blocks share a CU.  The tiles go longest first,
+// then the rest shortest first: a CU's two blocks then add up to about the same work.
+// Bound: the f32 matrix cores and the key / value re-reads (every block reads its whole context).
+// 1000 tokens behind 536 (8.5 GFLOP): 171 -> 118 us, 72 TFLOP/s of the 157 nominal; 512 from 0: 45 -> 40;
+// 1024 behind 4096: 579 -> 422 (the call, with the norm and rotary launch before it).
 constexpr int kRows = 16;          // query rows per block
-constexpr int kAW = 4;             // waves per block
-constexpr int kAT = 64 * kAW;
-constexpr int kKvLd = kHdP + 4;    // padded key / value / query rows in LDS (rows 4 banks apart)
-__global__ __launch_bounds__(kAT, 1) void attn_prefill_kernel(const AttnPrefill a) {
-  __shared__ __align__(16) float Qs[kRows][kKvLd];
-  __shared__ __align__(16) float KV[kAW][2][16][kKvLd];  // per wave: key tile, value tile
+constexpr int kKvLd = kHdP + 4;    // padded rows in LDS (rows 4 banks apart)
+template <int kAW>  // waves per block
+__global__ __launch_bounds__(64 * kAW, kAW == 4 ? 2 : 1) void attn_prefill_kernel(const AttnPrefill a) {
+  constexpr int kAT = 64 * kAW;
+  // the block's query rows, then (they are done by then) the waves' outputs [kAW][kRows][kKvLd]
+  __shared__ __align__(16) float sm[kAW * kRows * kKvLd];
   __shared__ float Mw[kAW][kRows], Lw[kAW][kRows];
+  float (*Qs)[kKvLd] = reinterpret_cast<float (*)[kKvLd]>(sm);
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c16 = l & 15, g = l >> 4;
   const int rep = a.nh / a.nkv, QT = kRows / rep;
-  const int gk = blockIdx.x % a.nkv, tile = blockIdx.x / a.nkv;
+  const int gk = blockIdx.x % a.nkv, ti = blockIdx.x / a.nkv, half = (a.sq.tiles + 1) / 2;
+  const int tile = ti < half ? a.sq.tiles - 1 - ti : ti - half;
   const PfSeq sq = pf_seq<&PfSeqs::tile0>(a.sq, tile);
   const int qt = tile - sq.tile0, tb = sq.tb, T = sq.T, p0 = sq.p0;
   const int t = qt * QT + c16 / rep;  // the lane's query row c16: token t of the sequence
   const int lim = p0 + min(t, T - 1);  // last key row c16 may see (rows past T are discarded)
   const int tmax_blk = min(T, (qt + 1) * QT) - 1;
   const int nkeys = p0 + tmax_blk + 1;
-  for (int e = tid; e < kRows * kHdP / 4; e += kAT) {
-    const int r = e >> 6, d = (e & 63) * 4;
-    const int tr = tb + min(qt * QT + r / rep, T - 1), hr = gk * rep + r % rep;
-    *(q35_f32x4*)&Qs[r][d] = *(const q35_f32x4*)(a.qbuf + ((int64_t)tr * a.nh + hr) * kHdP + d);
-  }
   const int64_t cache = ((int64_t)sq.slot * a.nkv + gk) * a.tmax * kHdP;
-  const float* Kg = a.kc + cache;
-  const float* Vg = a.vc + cache;
-  float (*Kt)[kKvLd] = KV[w][0];
-  float (*Vt)[kKvLd] = KV[w][1];
-  q35_f32x4 nk[16], nv[16];  // the next tile: key row u, dims 4 l .. 4 l + 3
-  auto load_tile = [&](int k0) {
+  const float* Kg = a.kc + cache + 4 * g;
+  const float* Vg = a.vc + cache + 4 * c16;
+  mfma_f4 kv[16], vv[4][4];  // keys: row c16, dims 16 kk + 4 g ..; values: row 4 g + mm, dims 64 q + 4 c16 ..
+  auto load_k = [&](int k0) {
+    const float* p = Kg + (int64_t)min(k0 + c16, nkeys - 1) * kHdP;
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int kj = min(k0 + u, nkeys - 1);
-      nk[u] = *(const q35_f32x4*)(Kg + (int64_t)kj * kHdP + 4 * l);
-      nv[u] = *(const q35_f32x4*)(Vg + (int64_t)kj * kHdP + 4 * l);
+    for (int kk = 0; kk < 16; ++kk) kv[kk] = *(const Q35_GLOBAL mfma_f4*)(p + 16 * kk);
+  };
+  auto load_v = [&](int k0) {
+#pragma unroll
+    for (int mm = 0; mm < 4; ++mm) {
+      const float* p = Vg + (int64_t)min(k0 + 4 * g + mm, nkeys - 1) * kHdP;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) vv[mm][q] = *(const Q35_GLOBAL mfma_f4*)(p + 64 * q);
     }
   };
+  // (the queries' loads first: loads return in order)
+  constexpr int kQV = kRows * kHdP / 4 / kAT;
+  mfma_f4 qv[kQV];
+#pragma unroll
+  for (int u = 0; u < kQV; ++u) {
+    const int e = tid + u * kAT, r = e >> 6, d = (e & 63) * 4;
+    const int tr = tb + min(qt * QT + r / rep, T - 1), hr = gk * rep + r % rep;
+    qv[u] = *(const Q35_GLOBAL mfma_f4*)(a.qbuf + ((int64_t)tr * a.nh + hr) * kHdP + d);
+  }
+  int k0 = 16 * w;
+  if (k0 < nkeys) {
+    load_k(k0);
+    load_v(k0);
+  }
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int u = 0; u < kQV; ++u) *(mfma_f4*)&Qs[(tid + u * kAT) >> 6][((tid + u * kAT) & 63) * 4] = qv[u];
   mfma_f4 o[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) o[i] = mfma_f4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, lsum = 0.f;
   const float sl2 = a.scale * 1.44269504088896341f;
-  int k0 = 16 * w;
-  if (k0 < nkeys) load_tile(k0);
   __syncthreads();  // Qs
   for (; k0 < nkeys; k0 += 16 * kAW) {
-    // (the wave's reads of its slot in the previous tile precede these stores: LDS is in order)
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      *(q35_f32x4*)&Kt[u][4 * l] = nk[u];
-      *(q35_f32x4*)&Vt[u][4 * l] = nv[u];
-    }
-    if (k0 + 16 * kAW < nkeys) load_tile(k0 + 16 * kAW);
-    mfma_f4 sc = {0.f, 0.f, 0.f, 0.f};
+    const bool more = k0 + 16 * kAW < nkeys;
+    // two accumulators: consecutive products do not wait for each other's result
+    mfma_f4 sc0 = {0.f, 0.f, 0.f, 0.f}, sc1 = sc0;
 #pragma unroll
     for (int kk = 0; kk < kHdP / 16; ++kk) {
-      const mfma_f4 ka = *(const mfma_f4*)&Kt[c16][16 * kk + 4 * g];
       const mfma_f4 qb = *(const mfma_f4*)&Qs[c16][16 * kk + 4 * g];
 #pragma unroll
-      for (int mm = 0; mm < 4; ++mm) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[mm], qb[mm], sc, 0, 0, 0);
+      for (int mm = 0; mm < 4; mm += 2) {
+        sc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[kk][mm], qb[mm], sc0, 0, 0, 0);
+        sc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[kk][mm + 1], qb[mm + 1], sc1, 0, 0, 0);
+      }
     }
+    if (more) load_k(k0 + 16 * kAW);
+    asm volatile("" ::: "memory");
+    const mfma_f4 sc = sc0 + sc1;
     float sv[4], bm = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -791,19 +812,24 @@ __global__ __launch_bounds__(kAT, 1) void attn_prefill_kernel(const AttnPrefill 
     ps += __shfl_xor(ps, 32, 64);
     lsum = lsum * alpha + ps;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      o[i] *= alpha;
+    for (int i = 0; i < 16; ++i) o[i] *= alpha;
 #pragma unroll
-      for (int mm = 0; mm < 4; ++mm)
-        o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(Vt[4 * g + mm][16 * i + c16], p[mm], o[i], 0, 0, 0);
-    }
+    for (int mm = 0; mm < 4; ++mm)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[mm][i >> 2][i & 3], p[mm], o[i], 0, 0, 0);
+    if (more) load_v(k0 + 16 * kAW);
+    asm volatile("" ::: "memory");
   }
   // merge the waves' states (key 0, in wave 0's first tile, is visible to every row, so wave 0's
-  // maximum is finite)
+  // maximum is finite); register r of o[i] is dim 64 (i / 4) + 4 (4 g + r) + i % 4 of row c16
   __syncthreads();
-  float* Om = &KV[0][0][0][0];  // [kAW][kRows][kKvLd]
 #pragma unroll
-  for (int i = 0; i < 16; ++i) *(mfma_f4*)&Om[(w * kRows + c16) * kKvLd + 16 * i + 4 * g] = o[i];
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *(mfma_f4*)&sm[(w * kRows + c16) * kKvLd + 64 * q + 16 * g + 4 * r] =
+          mfma_f4{o[4 * q][r], o[4 * q + 1][r], o[4 * q + 2][r], o[4 * q + 3][r]};
   if (g == 0) {
     Mw[w][c16] = m;
     Lw[w][c16] = lsum;
@@ -811,7 +837,7 @@ __global__ __launch_bounds__(kAT, 1) void attn_prefill_kernel(const AttnPrefill 
   __syncthreads();
   const int q = tid >> 4, d0 = (tid & 15) * 16;
   const int hq = gk * rep + q % rep;
-  if (qt * QT + q / rep >= T) return;
+  if (tid >= 16 * kRows || qt * QT + q / rep >= T) return;
   const int tq = tb + qt * QT + q / rep;
   float M = Mw[0][q];
 #pragma unroll
@@ -828,7 +854,7 @@ __global__ __launch_bounds__(kAT, 1) void attn_prefill_kernel(const AttnPrefill 
   for (int d = 0; d < 16; d += 4) {
     q35_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ww = 0; ww < kAW; ++ww) acc += *(const q35_f32x4*)&Om[(ww * kRows + q) * kKvLd + d0 + d] * f[ww];
+    for (int ww = 0; ww < kAW; ++ww) acc += *(const q35_f32x4*)&sm[(ww * kRows + q) * kKvLd + d0 + d] * f[ww];
     const float4 gv = *(const float4*)(gate + d);
     *(float4*)(dst + d) = make_float4((acc[0] / L) * sigmoid_f(gv.x), (acc[1] / L) * sigmoid_f(gv.y),
                                       (acc[2] / L) * sigmoid_f(gv.z), (acc[3] / L) * sigmoid_f(gv.w));
@@ -931,7 +957,11 @@ int attn_prefill_launch(const AttnPrefill& a, hipStream_t st) {
   if ((a.ld_qg % 4) != 0 || (a.ld_out % 4) != 0) return fail(Q35_E_ALIGN, "attention prefill: row alignment");
   hipLaunchKernelGGL(attn_prefill_prep_kernel, dim3(a.sq.rows * (a.nh + a.nkv)), dim3(kPT), 0, st, a);
   Q35_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(attn_prefill_kernel, dim3(a.sq.tiles * a.nkv), dim3(kAT), 0, st, a);
+  // few query tiles leave CUs without a block: twice the waves on each tile's keys then (16 tokens
+  // behind 3000: 151 -> 145 us, 16 tokens from 0: 15 -> 13.4)
+  const int nb = a.sq.tiles * a.nkv;
+  if (nb <= 128) hipLaunchKernelGGL(attn_prefill_kernel<8>, dim3(nb), dim3(512), 0, st, a);
+  else hipLaunchKernelGGL(attn_prefill_kernel<4>, dim3(nb), dim3(256), 0, st, a);
   Q35_HIP_TRY(hipGetLastError());
   return Q35_OK;
 }
