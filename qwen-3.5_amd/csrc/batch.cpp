@@ -42,6 +42,9 @@ struct q35_batch {
   float *gu = nullptr;     // gate | up rows [B][2 ffn], and a second copy for two split partials
   float *o_raw = nullptr, *attn = nullptr, *logits = nullptr, *pv = nullptr, *part = nullptr, *invf = nullptr;
   float* words = nullptr;  // counted split-K words of the projections (zero between launches)
+  // the matrix-core row path (dv = 128): normalised rows, the gates [B][2 heads], their partials
+  bool rows = false;
+  float *xn = nullptr, *bg = nullptr, *aux_part = nullptr;
   _Float16* split16 = nullptr;  // the lm_head's split input rows (hi, lo) of one row group
   q35::fx_t* ss = nullptr;   // RMSNorm statistics [2 layers + 1][B]
   q35::fx_t* gates = nullptr;  // DeltaNet gate sums [layers][B][32] (follows ss)
@@ -93,8 +96,10 @@ void bdestroy(q35_batch* b) {
 
 hipStream_t bpick(q35_batch* b, void* s) { return s ? static_cast<hipStream_t>(s) : b->own_stream; }
 
-// One decode step of all B rows (the launch sequence a graph captures).
-int batch_step_launch(q35_batch* bt, hipStream_t st) {
+// The layers' launches with the residual adds and norm statistics inside the projections
+// (mb_launch), for up to 4 rows and for
+// value heads other than 128 wide.
+int batch_layers_counted(q35_batch* bt, hipStream_t st) {
   const q35_model* m = bt->m;
   const q35_dims& d = m->d;
   const int B = bt->B, H = d.hidden, F = d.ffn, NL = d.n_layers;
@@ -104,11 +109,6 @@ int batch_step_launch(q35_batch* bt, hipStream_t st) {
   const int ldqg = ah * hd * 2, kvw = kvh * hd;
   int rc;
   std::vector<int32_t> gu_two((B + kRowGroup - 1) / kRowGroup, 0);  // gate|up left two partials
-  // embedding rows + the first norm's statistic; clears every other statistic and gate sum
-  if ((rc = batch_embed_f32_launch(m->embed.q, m->embed.s, H, bt->token, bt->prompt, bt->tmax, bt->plen, bt->pos, bt->h,
-                                   bt->ss, bt->ss + B, (int64_t)2 * NL * B + (int64_t)NL * B * kGateLd,
-                                   ws_counters(bt->ws) + kWsErrWord, B, st)))
-    return rc;
   auto base = [&](MbCall& c, int M) {
     c.M = M; c.eps = d.eps;
     c.part = bt->part; c.part_floats = bt->part_floats; c.ctr = bt->mb_ctr; c.nctr = kMbCounters;
@@ -199,6 +199,112 @@ int batch_step_launch(q35_batch* bt, hipStream_t st) {
       if ((rc = mb_launch(c, st))) return rc;
     }
   }
+  return Q35_OK;
+}
+
+// The layers' launches on the multi-row matvec (mvm.hip): every projection leaves its K splits as
+// plain partials; the next launch adds them, with the element-wise work between two projections in
+// it: the residual add and the RMSNorm (rms_rows), the SwiGLU, or the gates' activations.  The 2B step
+// at 8 / 16 / 24 / 32 rows: 1433 / 1797 / 2853 / 3065 us with batch_layers_counted, which stages,
+// normalises and re-scales its input rows in every column block and hands K splits over through
+// returning atomics; 1378 / 1632 / 2119 / 2385 here.
+int batch_layers_rows(q35_batch* bt, hipStream_t st) {
+  const q35_model* m = bt->m;
+  const q35_dims& d = m->d;
+  const int B = bt->B, H = d.hidden, F = d.ffn, NL = d.n_layers;
+  const int nh = d.lin_heads, vdim = nh * d.lin_dv, conv_dim = 2 * nh * d.lin_dk + vdim, ldq = (int)bt->proj_n;
+  const int ah = d.attn_heads, kvh = d.kv_heads, hd = d.head_dim;
+  const int ldqg = ah * hd * 2, kvw = kvh * hd;
+  uint32_t* err = ws_counters(bt->ws) + kWsErrWord;
+  int rc;
+  auto seg = [](const q35_model::Q8& w, const q35_model::Mb& mb) { return MvmSeg{mb.qs, mb.s, w.cols, 0}; };
+  auto base = [&](MvmCall& c, int K, const float* x, int ldx, int r0) {
+    c.M = std::min(kRowGroup, B - r0); c.K = K; c.x = x + (size_t)r0 * ldx; c.ldx = ldx; c.eps = d.eps;
+    c.part = bt->part; c.part_floats = bt->part_floats; c.err = err; c.stream_order = true;
+  };
+  // h += the residual projection c's partials, xn = RMSNorm(h) with the next norm's weights
+  auto residual = [&](MvmCall& c, int r0, const float* w) -> int {
+    int32_t ns = 0;
+    c.nsplit_out = &ns;
+    const int e = mvm_launch(c, st);
+    return e ? e : rms_rows_launch(bt->h + (size_t)r0 * H, H, c.M, H, w, d.eps, bt->xn + (size_t)r0 * H, H, st, nullptr,
+                                   bt->part, ns, (int64_t)c.M * H, H, nullptr, err);
+  };
+  if ((rc = rms_rows_launch(bt->h, H, B, H, m->layers[0].in_norm, d.eps, bt->xn, H, st, nullptr, nullptr, 0, 0, 0, nullptr, err)))
+    return rc;
+  for (int l = 0; l < NL; ++l) {
+    const q35_model::Layer& L = m->layers[l];
+    const q35_model::MbLayer& W = m->mb[l];
+    for (int r0 = 0; r0 < B; r0 += kRowGroup) {
+      MvmCall c;
+      base(c, H, bt->xn, H, r0);
+      c.y = bt->proj + (size_t)r0 * ldq; c.ldy = ldq;
+      if (!L.full) {
+        c.nseg = 2; c.seg[0] = seg(L.qkv, W.qkv); c.seg[1] = seg(L.z, W.z);
+        c.aux_wb = L.w_b; c.aux_wa = L.w_a; c.aux_nh = nh; c.a_log = L.a_log; c.dt_bias = L.dt_bias;
+        c.bg = bt->bg + (size_t)r0 * 2 * nh; c.aux_part = bt->aux_part;
+      } else {
+        c.nseg = 3; c.seg[0] = seg(L.q, W.q); c.seg[1] = seg(L.k, W.k); c.seg[2] = seg(L.v, W.v);
+      }
+      if ((rc = mvm_launch(c, st))) return rc;
+    }
+    if (!L.full) {
+      GdnCall g;
+      g.qkv = bt->proj; g.ld_qkv = ldq; g.bg = bt->bg; g.ld_bg = 2 * nh;
+      g.conv_state = bt->conv[l]; g.conv_w = L.conv_w; g.S = bt->rec[l]; g.o = bt->o_raw; g.ld_o = vdim;
+      g.B = B; g.nh = nh; g.dk = d.lin_dk; g.dv = d.lin_dv; g.conv_k = d.conv_k; g.head_ctr = bt->gdn_ctr;
+      if ((rc = gdn_step_launch(g, st))) return rc;
+    } else {
+      AttnCall a;
+      a.qg = bt->proj; a.ld_qg = ldq; a.k = bt->proj + ldqg; a.v = bt->proj + ldqg + kvw; a.ld_kv = ldq;
+      a.qnw = L.q_norm; a.knw = L.k_norm; a.eps = d.eps;
+      a.rcos = m->rope_cos; a.rsin = m->rope_sin; a.rot = d.rot_dim;
+      a.kc = bt->kc[l]; a.vc = bt->vc[l]; a.tmax = bt->tmax; a.pos = bt->pos;
+      a.out = bt->attn; a.ld_out = ah * hd; a.B = B; a.nh = ah; a.nkv = kvh; a.hd = hd;
+      if ((rc = attn_launch(a, bt->ws, bt->ws_bytes, st))) return rc;
+    }
+    for (int r0 = 0; r0 < B; r0 += kRowGroup) {
+      MvmCall c;
+      if (!L.full) {
+        base(c, vdim, bt->o_raw, vdim, r0);
+        c.z = bt->proj + (size_t)r0 * ldq + conv_dim; c.ldz = ldq; c.pw = L.norm_w;
+        c.seg[0] = seg(L.out, W.out);
+      } else {
+        base(c, ah * hd, bt->attn, ah * hd, r0);
+        c.seg[0] = seg(L.o, W.o);
+      }
+      c.nseg = 1;
+      if ((rc = residual(c, r0, L.post_norm))) return rc;
+    }
+    for (int r0 = 0; r0 < B; r0 += kRowGroup) {
+      MvmCall c;
+      base(c, H, bt->xn, H, r0);
+      c.nseg = 2; c.seg[0] = seg(L.gate, W.gate); c.seg[1] = seg(L.up, W.up);
+      c.y = bt->gu + (size_t)r0 * F; c.ldy = F; c.swiglu = 1;
+      if ((rc = mvm_launch(c, st))) return rc;
+    }
+    for (int r0 = 0; r0 < B; r0 += kRowGroup) {
+      MvmCall c;
+      base(c, F, bt->gu, F, r0);
+      c.nseg = 1; c.seg[0] = seg(L.down, W.down);
+      if ((rc = residual(c, r0, l + 1 < NL ? m->layers[l + 1].in_norm : m->final_norm))) return rc;
+    }
+  }
+  return Q35_OK;
+}
+
+// One decode step of all B rows (the launch sequence a graph captures).
+int batch_step_launch(q35_batch* bt, hipStream_t st) {
+  const q35_model* m = bt->m;
+  const q35_dims& d = m->d;
+  const int B = bt->B, H = d.hidden, NL = d.n_layers;
+  int rc;
+  // embedding rows + the first norm's statistic; clears every other statistic and gate sum
+  if ((rc = batch_embed_f32_launch(m->embed.q, m->embed.s, H, bt->token, bt->prompt, bt->tmax, bt->plen, bt->pos, bt->h,
+                                   bt->ss, bt->ss + B, (int64_t)2 * NL * B + (int64_t)NL * B * kGateLd,
+                                   ws_counters(bt->ws) + kWsErrWord, B, st)))
+    return rc;
+  if ((rc = bt->rows ? batch_layers_rows(bt, st) : batch_layers_counted(bt, st))) return rc;
   // final RMSNorm and the tied lm_head (model.rs:113-129) for every row
   for (int r0 = 0; r0 < B; r0 += kRowGroup)
     if ((rc = mb_lm_head_launch(m->embed_lm, m->embed_scale_t, d.vocab, H, bt->h + (size_t)r0 * H, H, m->final_norm, d.eps,
@@ -458,10 +564,18 @@ int q35_batch_create(q35_model* m, int32_t B, int32_t tmax, q35_batch** out) {
     b->part_floats = std::max(b->part_floats, mb_part_floats(kn[1] / 64, kn[0], M0));
     b->word_floats = std::max(b->word_floats, mb_word_floats(kn[1] / 64, M0));
   }
+  // (at 2 and 4 rows the four more launches per layer cost as much as they save: 1228 against 1254 us
+  // and 1281 against 1288)
+  b->rows = d.lin_dv == 128 && B > 4;
+  for (const auto& kn : shapes)
+    b->part_floats = std::max(b->part_floats, mvm_part_floats(M0, kn[0], kn[1], &kn == &shapes[1]));
   fx_t* stats = nullptr;
   if ((rc = balloc_t(b, "norm_stats", (size_t)(2 * NL + 1) * B + (size_t)NL * B * kGateLd, &stats))) return bail(rc);
   b->ss = stats;
   b->gates = stats + (size_t)(2 * NL + 1) * B;
+  if (b->rows && ((rc = balloc_t(b, "xn", (size_t)B * H, &b->xn)) || (rc = balloc_t(b, "gates", (size_t)B * 2 * nh, &b->bg)) ||
+                  (rc = balloc_t(b, "gate_partials", mvm_aux_floats(M0, H, nh), &b->aux_part))))
+    return bail(rc);
   if ((rc = balloc_t(b, "h", (size_t)B * H, &b->h)) || (rc = balloc_t(b, "proj", (size_t)B * b->proj_n, &b->proj)) ||
       (rc = balloc_t(b, "gu", (size_t)2 * B * 2 * F, &b->gu)) || (rc = balloc_t(b, "lm_split16", (size_t)2 * kRowGroup * H, &b->split16)) ||
       (rc = balloc_t(b, "lm_invf", kRowGroup, &b->invf)) ||

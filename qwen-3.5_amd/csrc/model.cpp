@@ -397,7 +397,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
   for (int l = 0; l < d.n_layers; ++l) {
     const q35_model::Layer& L = m->layers[l];
     const q35_model::MbLayer& W = m->mb[l];
-    if ((rc = rms_rows_launch(m->pf_x, H, T, H, L.in_norm, d.eps, m->pf_xn, H, st, m->pf_aux, m->pf_part, pend,
+    if ((rc = rms_rows_launch(m->pf_x, H, T, H, L.in_norm, d.eps, m->pf_xn, H, st, m->pf_aux, pend > 1 ? m->pf_part : nullptr, pend,
                               pstride, H)))
       return rc;
     pend = 1;
@@ -447,7 +447,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
       o.part = m->pf_part; o.part_floats = gemm_part_floats(m->pf_cap, d.hidden); o.aux = m->pf_aux;
       if ((rc = gemm_launch(o, st))) return rc;
     }
-    if ((rc = rms_rows_launch(m->pf_x, H, T, H, L.post_norm, d.eps, m->pf_xn, H, st, m->pf_aux, m->pf_part, pend,
+    if ((rc = rms_rows_launch(m->pf_x, H, T, H, L.post_norm, d.eps, m->pf_xn, H, st, m->pf_aux, pend > 1 ? m->pf_part : nullptr, pend,
                               pstride, H, m->pf_act_max)))
       return rc;
     pend = 1;

@@ -37,6 +37,7 @@ typedef q35_h8 h8;
 constexpr int kAuxRows = 128;  // K rows per gate-projection block
 constexpr int kAuxLd = 132;    // its padded f32 x row in LDS
 
+enum { LAY_KN = 0, LAY_SO = 1 };  // KN / tile-major, or the batched decoder's stream-order records
 struct MvmSegArg {
   const int8_t* q;
   const float* s;
@@ -127,7 +128,7 @@ Q35_DEV void mvm_aux(const MvmArgs& a, int ab, float* xs) {
   }
 }
 
-template <int MT, int NS, int NW, bool GATED>
+template <int MT, int NS, int NW, bool GATED, int LAY>
 __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
   constexpr int RW = 32 * NS;               // K rows per wave
   constexpr int LD = 68;                    // padded row of the reduction buffer
@@ -152,16 +153,20 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
   const int lcb = cb - sg.cb0;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
   const int k0 = (split * NW + w) * RW;
-  // tile-major: tile lcb / 4 starts at row (lcb / 4) * K of a 256-column matrix
+  // tile-major: tile lcb / 4 starts at row (lcb / 4) * K of a 256-column matrix.  Stream order: per
+  // 32-row step 2 KB, the lane's operands of column tiles 0, 1 at 16 lane and of 2, 3 at 1024 + 16
+  // lane (column 16 nt + c there); scales [cb][K].
   const size_t trow = sg.tiled ? (size_t)(lcb >> 2) * a.K : 0;
-  const int8_t* wb = sg.q + trow * sg.ldq + (sg.tiled ? lcb & 3 : lcb) * 64 + 4 * c;
-  const float* sb = sg.s + trow * sg.lds + (sg.tiled ? lcb & 3 : lcb);
+  const int8_t* wb = LAY == LAY_SO ? sg.q + (size_t)lcb * a.K * 64 + 16 * lane
+                                   : sg.q + trow * sg.ldq + (sg.tiled ? lcb & 3 : lcb) * 64 + 4 * c;
+  const float* sb = LAY == LAY_SO ? sg.s + (size_t)lcb * a.K : sg.s + trow * sg.lds + (sg.tiled ? lcb & 3 : lcb);
+  const int lds = LAY == LAY_SO ? 1 : sg.lds;
 
   // every load of the wave, issued in the order of use; rows past K repeat its last 8 (their y
   // is set to zero)
   float sv[(RW + 63) / 64];
 #pragma unroll
-  for (int i = 0; i < (RW + 63) / 64; ++i) sv[i] = ldg(sb + (size_t)min(k0 + 64 * i + lane, a.K - 1) * sg.lds);
+  for (int i = 0; i < (RW + 63) / 64; ++i) sv[i] = ldg(sb + (size_t)min(k0 + 64 * i + lane, a.K - 1) * lds);
   f4 xv[NS][MT][2], zv[GATED ? NS : 1][MT][2], pv[GATED ? NS : 1][2];
   int kk[NS];
 #pragma unroll
@@ -184,9 +189,20 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
   }
   uint32_t wv[NS][8];
 #pragma unroll
-  for (int st = 0; st < NS; ++st)
+  for (int st = 0; st < NS; ++st) {
+    if constexpr (LAY == LAY_SO) {
+      const int8_t* p = wb + (size_t)min(k0 + 32 * st, a.K - 32) * 64;
+      const q35_u32x4 w0 = ldg16v_nt(p), w1 = ldg16v_nt(p + 1024);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) wv[st][j] = ldg_nt((const uint32_t*)(wb + (size_t)(kk[st] + j) * sg.ldq));
+      for (int j = 0; j < 4; ++j) {
+        wv[st][j] = w0[j];
+        wv[st][4 + j] = w1[j];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) wv[st][j] = ldg_nt((const uint32_t*)(wb + (size_t)(kk[st] + j) * sg.ldq));
+    }
+  }
   __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to their uses)
 
   // the wave's scales through its own LDS rows (no other wave reads them)
@@ -266,7 +282,16 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) b[q][mt] = __builtin_bit_cast(h8, q35_u32x4{p[q][0], p[q][1], p[q][2], p[q][3]});
     }
-    const h8 aw[4] = {col8<0>(wv[st]), col8<1>(wv[st]), col8<2>(wv[st]), col8<3>(wv[st])};
+    h8 aw[4];
+    if constexpr (LAY == LAY_SO) {
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) aw[nt] = a8_from(wv[st][2 * nt], wv[st][2 * nt + 1]);
+    } else {
+      aw[0] = col8<0>(wv[st]);
+      aw[1] = col8<1>(wv[st]);
+      aw[2] = col8<2>(wv[st]);
+      aw[3] = col8<3>(wv[st]);
+    }
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
@@ -285,14 +310,17 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] += accs[nt][mt];
 
-  // lane holds column 16 g + 4 r + nt of row 16 mt + c in acc[nt][mt][r]; the waves' sums meet in
-  // LDS (2^-e undone first: it differs per wave) and are added in wave order
+  // lane holds column 16 g + 4 r + nt (stream order: 16 nt + 4 g + r) of row 16 mt + c in
+  // acc[nt][mt][r]; the waves' sums meet in LDS (2^-e undone first: it differs per wave) and are
+  // added in wave order
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      *(f4*)&red[(w * 16 * MT + 16 * mt + c) * LD + 16 * g + 4 * r] =
-          f4{acc[0][mt][r], acc[1][mt][r], acc[2][mt][r], acc[3][mt][r]} * inv[mt];
+    for (int r = 0; r < 4; ++r) {
+      float* rr = &red[(w * 16 * MT + 16 * mt + c) * LD];
+      if constexpr (LAY == LAY_SO) *(f4*)(rr + 16 * r + 4 * g) = acc[r][mt] * inv[mt];
+      else *(f4*)(rr + 16 * g + 4 * r) = f4{acc[0][mt][r], acc[1][mt][r], acc[2][mt][r], acc[3][mt][r]} * inv[mt];
+    }
   __syncthreads();
   const int ldp = 64 * a.ncb;
 #pragma unroll
@@ -406,12 +434,17 @@ MvmPlan mvm_plan(int ncb, int K, bool gated) {
   return p;
 }
 
-template <int MT, bool GATED>
+template <int MT, bool GATED, int LAY>
 const void* mvm_fn(const MvmPlan& p) {
-  if (p.ns == 4 && p.nw == 4) return (const void*)mvm_kernel<MT, 4, 4, GATED>;
-  if (p.ns == 4) return (const void*)mvm_kernel<MT, 4, 2, GATED>;
-  if constexpr (!GATED) return (const void*)mvm_kernel<MT, 2, 2, false>;
+  if (p.ns == 4 && p.nw == 4) return (const void*)mvm_kernel<MT, 4, 4, GATED, LAY>;
+  if (p.ns == 4) return (const void*)mvm_kernel<MT, 4, 2, GATED, LAY>;
+  if constexpr (!GATED) return (const void*)mvm_kernel<MT, 2, 2, false, LAY>;
   return nullptr;
+}
+template <int LAY>
+const void* mvm_pick(const MvmPlan& p, int M, bool gated) {
+  if (M <= 16) return gated ? mvm_fn<1, true, LAY>(p) : mvm_fn<1, false, LAY>(p);
+  return gated ? mvm_fn<2, true, LAY>(p) : mvm_fn<2, false, LAY>(p);
 }
 
 }  // namespace
@@ -429,7 +462,7 @@ bool mvm_ok(const float* x, int32_t ldx, int32_t K) {
 int mvm_launch(const MvmCall& c, hipStream_t st) {
   if (c.M < 1 || c.M > kMvmRows || c.nseg < 1 || c.nseg > kMvmMaxSeg) return fail(Q35_E_SHAPE, "mvm: bad rows or segments");
   if (!mvm_ok(c.x, c.ldx, c.K)) return fail(Q35_E_ALIGN, "mvm: K % 32 and 16-byte aligned rows required");
-  if (!c.y || !c.part || !c.err) return fail(Q35_E_ARG, "mvm: null pointer");
+  if ((!c.y && !c.nsplit_out) || !c.part || !c.err) return fail(Q35_E_ARG, "mvm: null pointer");
   const bool gated = c.z != nullptr;
   if (gated && (!c.pw || c.K % 128 || c.ldz % 4 || (reinterpret_cast<uintptr_t>(c.z) & 15) ||
                 (reinterpret_cast<uintptr_t>(c.pw) & 15)))
@@ -454,11 +487,14 @@ int mvm_launch(const MvmCall& c, hipStream_t st) {
     a.aux_wb = c.aux_wb; a.aux_wa = c.aux_wa; a.aux_nh = c.aux_nh; a.aux_part = c.aux_part;
     r.aux = c.aux_part; r.naux = a.naux; r.nh = c.aux_nh; r.alog = c.a_log; r.dtb = c.dt_bias; r.bg = c.bg;
   }
-  const void* k = c.M <= 16 ? (gated ? mvm_fn<1, true>(p) : mvm_fn<1, false>(p))
-                            : (gated ? mvm_fn<2, true>(p) : mvm_fn<2, false>(p));
+  const void* k = c.stream_order ? mvm_pick<LAY_SO>(p, c.M, gated) : mvm_pick<LAY_KN>(p, c.M, gated);
   void* params[] = {&a};
   Q35_HIP_TRY(hipLaunchKernel(k, dim3((unsigned)(a.naux + ncb * p.nsplit)), dim3(64 * p.nw), params, 0, st));
   Q35_HIP_TRY(hipGetLastError());
+  if (c.nsplit_out) {
+    *c.nsplit_out = p.nsplit;
+    return Q35_OK;
+  }
   r.part = c.part; r.nsplit = p.nsplit; r.M = c.M; r.N = 64 * ncb; r.y = c.y; r.ldy = c.ldy;
   r.swiglu = c.swiglu; r.clear = c.clear; r.err = c.err;
   const int64_t nout = (int64_t)c.M * (c.swiglu ? r.N / 2 : r.N) / 4;

@@ -56,8 +56,8 @@ Q35_DEV void block_max256_store(float v, float* sh, float* dst) {
 }
 
 // y[m] = x[m] * rsqrt(mean(x[m]^2) + eps) * (1 + w)  (text_modules.rs:800-808).  amax (optional):
-// max |y[m]| of each row, the row maxima the matrix-core GEMM that consumes y needs.  With nsplit >
-// 1, x[m] is first replaced by ((part_0 + part_1) + ...) + x[m], the K splits of the GEMM that
+// max |y[m]| of each row, the row maxima the matrix-core GEMM that consumes y needs.  With part,
+// x[m] is first replaced by ((part_0 + part_1) + ...) + x[m], the K splits of the GEMM that
 // accumulates into x added in split order as its reduction kernel would.  clear (optional): set to
 // zero per row (the next GEMM's SwiGLU row maxima, raised by atomics).  Rows of up to
 // kRmsHeld * 4 * 256 floats (K a multiple of 4, rows 16-byte aligned) stay in registers between
@@ -75,7 +75,8 @@ Q35_DEV float4 sum_parts(const float* p, int64_t stride) {
 }
 __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K, const float* w, float eps,
                                                        float* y, int ldy, float* amax, const float* part,
-                                                       int nsplit, int64_t sstride, int ldp, float* clear) {
+                                                       int nsplit, int64_t sstride, int ldp, float* clear,
+                                                       uint32_t* err) {
   __shared__ float sh[4];
   const int m = blockIdx.x;
   if (clear && threadIdx.x == 0) clear[m] = 0.f;
@@ -85,7 +86,7 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
   float mx = 0.f;
   if (K <= kRmsHeld * 4 * kPT && (K & 3) == 0 &&
       ((reinterpret_cast<uintptr_t>(xr) | reinterpret_cast<uintptr_t>(yr) | reinterpret_cast<uintptr_t>(w) |
-        reinterpret_cast<uintptr_t>(pr)) & 15) == 0 && (nsplit <= 1 || (sstride & 3) == 0)) {
+        reinterpret_cast<uintptr_t>(pr)) & 15) == 0 && (!pr || (sstride & 3) == 0)) {
     float4 v[kRmsHeld];
     float ss = 0.f;
 #pragma unroll
@@ -93,16 +94,18 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
       const int k = 4 * (threadIdx.x + u * kPT);
       v[u] = k < K ? *(const float4*)(xr + k) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    if (nsplit > 1) {
+    if (pr) {
 #pragma unroll
       for (int u = 0; u < kRmsHeld; ++u) {
         const int k = 4 * (threadIdx.x + u * kPT);
         if (k < K) {
           float4 t;
           switch (nsplit) {
+            case 1: t = sum_parts<1>(pr + k, sstride); break;
             case 2: t = sum_parts<2>(pr + k, sstride); break;
             case 4: t = sum_parts<4>(pr + k, sstride); break;
             case 8: t = sum_parts<8>(pr + k, sstride); break;
+            case 12: t = sum_parts<12>(pr + k, sstride); break;
             case 16: t = sum_parts<16>(pr + k, sstride); break;
             default:
               t = *(const float4*)(pr + k);
@@ -119,6 +122,8 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
 #pragma unroll
     for (int u = 0; u < kRmsHeld; ++u) ss += ((v[u].x * v[u].x + v[u].y * v[u].y) + v[u].z * v[u].z) + v[u].w * v[u].w;
     ss = block_sum256(ss, sh);
+    if (err && threadIdx.x == 0 && !fx_addable(ss))
+      __hip_atomic_fetch_or((Q35_GLOBAL uint32_t*)err, kWsErrRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const float r = rsqrt_f(ss * rcp_f((float)K) + eps);
 #pragma unroll
     for (int u = 0; u < kRmsHeld; ++u) {
@@ -135,7 +140,7 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
     float ss = 0.f;
     for (int k = threadIdx.x; k < K; k += kPT) {
       float v = xr[k];
-      if (nsplit > 1) {
+      if (pr) {
         float t = pr[k];
         for (int s = 1; s < nsplit; ++s) t += pr[s * sstride + k];
         v = t + v;
@@ -144,6 +149,8 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
       ss += v * v;
     }
     ss = block_sum256(ss, sh);
+    if (err && threadIdx.x == 0 && !fx_addable(ss))
+      __hip_atomic_fetch_or((Q35_GLOBAL uint32_t*)err, kWsErrRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const float r = rsqrt_f(ss * rcp_f((float)K) + eps);
     for (int k = threadIdx.x; k < K; k += kPT) {
       const float v = (xr[k] * r) * (1.0f + w[k]);
@@ -905,11 +912,11 @@ int last_rows_launch(const float* x, int ldx, int D, const PfArg& sq, float* h, 
 
 int rms_rows_launch(float* x, int ldx, int M, int K, const float* w, float eps, float* y, int ldy,
                     hipStream_t st, float* amax, const float* part, int nsplit, int64_t sstride, int ldp,
-                    float* clear) {
+                    float* clear, uint32_t* err) {
   if (M < 1) return Q35_OK;
-  if (nsplit > 1 && !part) return fail(Q35_E_ARG, "rms_rows: split partials missing");
+  if (part && nsplit < 1) return fail(Q35_E_ARG, "rms_rows: no splits in the partials");
   hipLaunchKernelGGL(rms_rows_kernel, dim3(M), dim3(kPT), 0, st, x, ldx, K, w, eps, y, ldy, amax,
-                     nsplit > 1 ? part : nullptr, nsplit, sstride, ldp, clear);
+                     part, nsplit, sstride, ldp, clear, err);
   Q35_HIP_TRY(hipGetLastError());
   return Q35_OK;
 }

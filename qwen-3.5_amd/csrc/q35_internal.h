@@ -457,6 +457,11 @@ struct MvmCall {
   const float* a_log = nullptr; const float* dt_bias = nullptr; float* bg = nullptr;
   float* aux_part = nullptr;                      // mvm_aux_floats
   float* part = nullptr; size_t part_floats = 0;  // mvm_part_floats
+  // the weights are the batched decoder's copies: records in stream order (mb_stream_launch), scales
+  // [N/64][K]
+  bool stream_order = false;
+  // set: no second launch; the partials [*nsplit_out][M][N] are the caller's to add, in split order
+  int32_t* nsplit_out = nullptr;
   int32_t clear = 0;  // zero the partials behind the call (a workspace shared by calls of other sizes)
   uint32_t* err = nullptr;                        // receives kWsErrRange
 };
@@ -737,12 +742,13 @@ int last_rows_launch(const float* x, int ldx, int D, const PfArg& sq, float* h, 
 // *p = v on the stream (a kernel, so it can sit in a captured graph)
 int store_i32_launch(int32_t* p, int32_t v, hipStream_t st);
 // y[m] = RMSNorm(x[m]) * (1 + w) for M rows of K
-// y = RMSNorm(x) (1 + w) per row; amax (optional): each row's max |y|.  part (optional, nsplit >
-// 1): K-split partial sums of a deferred GEMM that accumulates into x: x = ((part_0 + part_1) + ...)
-// + x is formed and written back to x first (split s, row m at part + s * sstride + m * ldp).
+// y = RMSNorm(x) (1 + w) per row; amax (optional): each row's max |y|.  part (optional):
+// nsplit K-split partial sums of a deferred GEMM that accumulates into x: x = ((part_0 + part_1) + ...)
+// + x is formed and written back to x first (split s, row m at part + s * sstride + m * ldp).  err
+// (optional): receives kWsErrRange when a row's sum of squares is not finite or >= 2^31.
 int rms_rows_launch(float* x, int ldx, int M, int K, const float* w, float eps, float* y, int ldy,
                     hipStream_t st, float* amax = nullptr, const float* part = nullptr, int nsplit = 1,
-                    int64_t sstride = 0, int ldp = 0, float* clear = nullptr);
+                    int64_t sstride = 0, int ldp = 0, float* clear = nullptr, uint32_t* err = nullptr);
 // [beta | g] rows of a prompt (x [T][ldx], softplus identity branch when its input exceeds 20)
 int gate_prompt_launch(const float* x, int ldx, int T, int K, const float* wb, const float* wa, const float* alog,
                        const float* dtb, int nh, float* out, hipStream_t st);

@@ -1,7 +1,8 @@
 """Prompts of a batch that share prompt passes: every row's ids equal a run of its own, where prompts
 of one token, of a chunk of 64, of 63 and 65, more prompts than one pass takes (32), and prompts longer
 than a pass (1024 tokens, then a rest that shares a pass with the next rows) meet; a second turn
-continues the rows' caches at different positions."""
+continues the rows' caches at different positions.  4 rows and 5 are the two sides of the choice
+between the decode step's launch sequences, 40 a second row group of 8."""
 import numpy as np
 import pytest
 
@@ -14,7 +15,7 @@ def dims():
     return q35.make_dims(hidden=512, ffn=1536, vocab=8192, n_layers=4, lin_heads=4, attn_heads=4, kv_heads=2)
 
 
-@pytest.mark.parametrize("lens", [[1, 64, 63, 65, 2, 3, 17], [5] * 40, [1100, 3, 70, 1025, 30]])
+@pytest.mark.parametrize("lens", [[9, 4, 30, 2], [1, 64, 63, 65, 2, 3, 17], [5] * 40, [1100, 3, 70, 1025, 30]])
 def test_batch_prompts_share_passes(lens):
     print(f"[batch prompts] {len(lens)} rows, longest {max(lens)}", flush=True)
     d, n_new, second = dims(), 6, 9
