@@ -14,6 +14,7 @@
 // to finish reduces the block results; the order is total, so the result does not depend on the
 // reduction order.
 #include "q35_internal.h"
+#include <algorithm>
 #include <climits>
 
 namespace q35 {
@@ -258,6 +259,178 @@ void launch_one(dim3 g, size_t lds, hipStream_t st, const NkArgs& a) {
   hipLaunchKernelGGL((nk_kernel<MR, CPW>), g, dim3(kThreads), lds, st, a);
 }
 
+// ---- 3 to 8 rows on the f16 matrix cores.  nk_kernel multiplies every weight by every row on the
+// vector ALUs, which bounds it from 2 rows on (248320 x 2048: 84 us at one row, 205 at 5, 364 at 8
+// with the final RMSNorm); here it is the table's stream again.  One block of 8 waves per CU stays for the
+// whole launch: its rows, split into three f16 values each (24 bits: q * x is exact before the f32
+// accumulation; the block scales belong to the output rows here and are applied to each 64-k sum),
+// are staged in LDS once.  A wave walks tiles of 64 table rows: lane (g, c) = (lane / 16, lane % 16)
+// takes bytes 16 g .. 16 g + 15 of every 64-byte block of row 16 nt + c, the A operands of two products
+// (k order permuted alike on both operands), four blocks ahead, across the tile's end.  The 64
+// rows' scales of 16 blocks pass through the wave's own LDS, loaded one group ahead.
+// 120 us at 2, 3 and 5 rows, 123 at 8 (4.4 TB/s), so 2 rows stay with nk_kernel.
+constexpr int kNmRows = 8, kNmWaves = 8, kNmT = 64 * kNmWaves, kNmKmax = 2048;
+constexpr int kNmSld = 68;  // padded row of 64 staged scales
+typedef q35_f32x4 nf4;
+size_t nkm_lds(int K) { return (size_t)3 * kNmRows * (K + 8) * 2 + (size_t)kNmWaves * 16 * kNmSld * 4; }
+__global__ __launch_bounds__(kNmT, 1) void nkm_kernel(const NkArgs a) {
+  extern __shared__ __align__(16) char nlds[];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
+  const int K = a.K, nb = K >> 6, ldx = K + 8;
+  _Float16* xs = reinterpret_cast<_Float16*>(nlds);                                  // [3][8][ldx]
+  float* sc = reinterpret_cast<float*>(nlds + (size_t)3 * kNmRows * ldx * 2) + w * 16 * kNmSld;  // [16][68]
+  const int ntiles = (a.N + 63) / 64, stride = gridDim.x * kNmWaves;
+  const int first = blockIdx.x * kNmWaves + w;
+  const int mine = first < ntiles ? (ntiles - first + stride - 1) / stride : 0, total = mine * nb;
+
+  // the ring of weight loads: (lt, lb) is the next block to request, past the end the last one again
+  q35_u32x4 wr[4][4];
+  int lt = min(first, ntiles - 1), lb = 0;
+  auto wload = [&](q35_u32x4 (&v)[4]) {
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+      v[nt] = *(const Q35_GLOBAL q35_u32x4*)(a.q + (size_t)min(64 * lt + 16 * nt + c, a.N - 1) * K + 64 * lb + 16 * g);
+    if (++lb == nb) {
+      lb = 0;
+      if (lt + stride < ntiles) lt += stride;
+    }
+  };
+  nf4 sr[4];
+  auto sload = [&](int t, int b0) {
+    const float* p = a.s + (size_t)min(64 * t + lane, a.N - 1) * nb;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sr[i] = *(const Q35_GLOBAL nf4*)(p + min(b0 + 4 * i, nb - 4));
+  };
+
+  // wave w stages row w (rows past M repeat the last one; their outputs are dropped)
+  float inv;
+  {
+    const int m = min(w, a.M - 1);
+    nf4 v[kNmKmax / 256], pw[kNmKmax / 256];
+    float ss = 0.f, mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < kNmKmax / 256; ++i) {
+      const int k = 256 * i + 4 * lane;
+      v[i] = k < K ? *(const Q35_GLOBAL nf4*)(a.x + (size_t)m * a.ldx + k) : nf4{0.f, 0.f, 0.f, 0.f};
+      pw[i] = (k < K && a.pro == PRO_RMS) ? *(const Q35_GLOBAL nf4*)(a.pw + k) : nf4{0.f, 0.f, 0.f, 0.f};
+    }
+    sload(lt, 0);
+    static_for<4>([&](auto d) { wload(wr[d]); });
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < kNmKmax / 256; ++i) ss += ((v[i][0] * v[i][0] + v[i][1] * v[i][1]) + v[i][2] * v[i][2]) + v[i][3] * v[i][3];
+    const float r = a.pro == PRO_RMS ? rsqrt_f(wave_sum(ss) / (float)K + a.eps) : 1.0f;
+#pragma unroll
+    for (int i = 0; i < kNmKmax / 256; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (a.pro == PRO_RMS) v[i][j] = (v[i][j] * r) * (1.0f + pw[i][j]);
+        mx = fmaxf(mx, fabsf(v[i][j]));
+      }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    float f;
+    split_scale(mx, f, inv);
+    if (lane == 0) sc[0] = inv;
+#pragma unroll
+    for (int i = 0; i < kNmKmax / 256; ++i) {
+      const int k = 256 * i + 4 * lane;
+      if (k >= K) break;
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        uint32_t p[3];
+        const float y0 = v[i][j] * f, y1 = v[i][j + 1] * f;
+        split3(y0, y1, p[0], p[1], p[2]);
+        // (an infinity has no remainder: its products are infinite, as in f32)
+        if (fabsf(y0) == INFINITY) { p[1] &= 0xffff0000u; p[2] &= 0xffff0000u; }
+        if (fabsf(y1) == INFINITY) { p[1] &= 0x0000ffffu; p[2] &= 0x0000ffffu; }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *(uint32_t*)&xs[(q * kNmRows + w) * ldx + k + j] = p[q];
+      }
+    }
+  }
+  __syncthreads();
+  inv = (sc - w * 16 * kNmSld)[(c & 7) * 16 * kNmSld];  // of row c
+  __syncthreads();
+  if (total == 0) return;
+
+  int ct = first, cb = 0;
+  nf4 acc[4];
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) acc[nt] = nf4{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < total; s0 += 4) {
+    static_for<4>([&](auto dc) {
+      constexpr int d = dc;
+      if (s0 + d < total) {
+        if ((cb & 15) == 0) {  // this group's scales to LDS [block][row], the next group's requested
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sc[(4 * i + j) * kNmSld + lane] = sr[i][j];
+          const bool more = cb + 16 < nb;
+          sload(more ? ct : min(ct + stride, ntiles - 1), more ? cb + 16 : 0);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+        }
+        // (a byte's place: k = 64 cb + 16 g + 8 h + j, products h = 0, 1)
+        q35_h8 b[3][2];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) b[q][h] = *(const q35_h8*)&xs[(q * kNmRows + (c & 7)) * ldx + 64 * cb + 16 * g + 8 * h];
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+          const q35_u32x4 wv = wr[d][nt] ^ 0x80808080u;  // int8 -> u = q + 128
+          const q35_h8 a0 = a8_from(wv[0], wv[1]), a1 = a8_from(wv[2], wv[3]);
+          nf4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int q = 2; q >= 0; --q) {  // smallest parts first
+            t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b[q][0], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, b[q][1], t, 0, 0, 0);
+          }
+          acc[nt] += t * *(const nf4*)&sc[(cb & 15) * kNmSld + 16 * nt + 4 * g];
+        }
+        wload(wr[d]);
+        asm volatile("" ::: "memory");  // (the ring's request stays here)
+        if (++cb == nb) {
+          cb = 0;
+          // lane holds rows 64 ct + 16 nt + 4 g + i of input row c
+          if (c < a.M) {
+            float* y = a.y + (size_t)c * a.ldy;
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const int n = 64 * ct + 16 * nt + 4 * g + i;
+                if (n < a.N) y[n] = acc[nt][i] * inv;
+              }
+          }
+          ct += stride;
+#pragma unroll
+          for (int nt = 0; nt < 4; ++nt) acc[nt] = nf4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+    });
+  }
+}
+
+// The calls nkm_kernel takes: f32 rows it can read in 16-byte pieces, whole groups of 4 scale blocks, and
+// enough table rows that its 8 waves per CU have work.
+bool nkm_ok(const NkCall& c) {
+  return c.M >= 3 && !c.xf && !c.argmax_out && c.K % 256 == 0 && c.K <= kNmKmax && c.N >= 32768 && c.ldx % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(c.x) & 15) == 0 && (reinterpret_cast<uintptr_t>(c.s) & 15) == 0 &&
+         (c.pro != PRO_RMS || (reinterpret_cast<uintptr_t>(c.pw) & 15) == 0) && nkm_lds(c.K) <= lds_per_block();
+}
+
+int nkm_cus() {
+  static int n = 0;
+  if (!n) {
+    int dev = 0, v = 0;
+    n = (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) ? v : 256;
+  }
+  return n;
+}
+
 template <int MR>
 void launch_mr(int cpw, dim3 g, size_t lds, hipStream_t st, const NkArgs& a) {
   if (cpw == 1) launch_one<MR, 1>(g, lds, st, a);
@@ -306,6 +479,13 @@ int nk_launch(const NkCall& c, void* ws, size_t ws_bytes, hipStream_t st) {
     a.counter = ws_counters(ws);
     a.part_v = reinterpret_cast<float*>(base);
     a.part_i = reinterpret_cast<int32_t*>(base + pb);
+  }
+  if (nkm_ok(c)) {
+    const size_t nl = nkm_lds(c.K);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(nkm_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)nl);
+    hipLaunchKernelGGL(nkm_kernel, dim3(std::min(nkm_cus(), (c.N + 64 * kNmWaves - 1) / (64 * kNmWaves))), dim3(kNmT), nl, st, a);
+    Q35_HIP_TRY(hipGetLastError());
+    return Q35_OK;
   }
   const size_t lds = (size_t)MR * c.K * sizeof(float);
   const int cpw = cpw_of(c.K);

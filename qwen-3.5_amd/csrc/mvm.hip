@@ -7,8 +7,8 @@
 // for each 8 rows and adds every column of every row with a 64-bit atomic; at 24 rows the MLP
 // spent 193 us on 38 MB of weights.  Here the products go to v_mfma_f32_16x16x32_f16 and the
 // K splits leave plain f32 partials that a second kernel adds in split order.  Measured, 2B layer
-// calls: MLP at 24 rows 192.6 -> 36.4 us, DeltaNet at 9 rows 85.6 -> 30.7, attention of 16 rows over
-// 8192-token caches 196 -> 108, q8_gemv 2048 x 6144 at 8 rows 35.0 -> 8.6.
+// calls: MLP at 24 rows 192.6 -> 33.6 us, DeltaNet at 9 rows 85.6 -> 27, the projections around the
+// attention of 16 rows 104 -> 24, q8_gemv 2048 x 6144 at 8 rows 35.0 -> 8.6.
 //
 // Arithmetic (f32-equivalent, as the other matrix-core paths): the int8 weight is exact in f16;
 // its block scale multiplies the input, y = x * s (f32), and y is carried whole, as three f16
@@ -69,18 +69,6 @@ Q35_DEV h8 col8(const uint32_t (&d)[8]) {
     r[j + 1] = p[1];
   }
   return r;
-}
-
-// y -> three f16 values (packed conversions, rounding toward zero) whose sum is y, each remainder
-// exact in f32: 24 bits down to 2^-14 of the largest value (2^14 after scaling)
-Q35_DEV void split3(float y0, float y1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  const q35_hf2 h = __builtin_amdgcn_cvt_pkrtz(y0, y1);
-  const float r0 = y0 - (float)h[0], r1 = y1 - (float)h[1];
-  const q35_hf2 m = __builtin_amdgcn_cvt_pkrtz(r0, r1);
-  const q35_hf2 l = __builtin_amdgcn_cvt_pkrtz(r0 - (float)m[0], r1 - (float)m[1]);
-  hi = __builtin_bit_cast(uint32_t, h);
-  mid = __builtin_bit_cast(uint32_t, m);
-  lo = __builtin_bit_cast(uint32_t, l);
 }
 
 // Gate projection (in_proj_b | in_proj_a, f32 [K][nh] each, kernels.rs:174-247): block ab sums
@@ -200,7 +188,9 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) wv[st][j] = ldg_nt((const uint32_t*)(wb + (size_t)(kk[st] + j) * sg.ldq));
+      for (int j = 0; j < 8; ++j)  // (64 bytes of a line: its other half belongs to the next column block,
+                                   // so no non-temporal hint: 36.4 -> 33.6 us for the MLP at 24 rows)
+        wv[st][j] = ldg((const uint32_t*)(wb + (size_t)(kk[st] + j) * sg.ldq));
     }
   }
   __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to their uses)

@@ -163,6 +163,18 @@ Q35_DEV void split2(float y0, float y1, uint32_t& hi, uint32_t& lo) {
   lo = __builtin_bit_cast(uint32_t, l);
 }
 
+// y -> three f16 values (packed conversions, rounding toward zero) whose sum is y, each remainder
+// exact in f32: 24 bits down to 2^-14 of the largest value (2^14 after scaling)
+Q35_DEV void split3(float y0, float y1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  const q35_hf2 h = __builtin_amdgcn_cvt_pkrtz(y0, y1);
+  const float r0 = y0 - (float)h[0], r1 = y1 - (float)h[1];
+  const q35_hf2 m = __builtin_amdgcn_cvt_pkrtz(r0, r1);
+  const q35_hf2 l = __builtin_amdgcn_cvt_pkrtz(r0 - (float)m[0], r1 - (float)m[1]);
+  hi = __builtin_bit_cast(uint32_t, h);
+  mid = __builtin_bit_cast(uint32_t, m);
+  lo = __builtin_bit_cast(uint32_t, l);
+}
+
 
 Q35_DEV void fx_add(fx_t* p, float v) {
   __hip_atomic_fetch_add((Q35_GLOBAL unsigned long long*)p, (unsigned long long)to_fx(v), __ATOMIC_RELAXED,

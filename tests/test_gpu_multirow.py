@@ -110,3 +110,37 @@ def test_one_row_layers_between_batches(hidden, ffn, heads):
         cs1, S1 = dev(cs[r:r + 1]), dev(S[r:r + 1])
         assert rel_l2(host(gdn.forward(x[r:r + 1], cs1, S1))[0], out_g[r]) <= 3e-6, r
         assert rel_l2(host(S1)[0], host(S3)[r]) <= 3e-6 and rel_l2(host(cs1)[0], host(cs3)[r]) <= 3e-6, r
+
+
+@pytest.mark.parametrize("N,K,M", [(32768, 256, 2), (32768 + 37, 512, 3), (70001, 1280, 5), (248320, 2048, 4),
+                                   (248320, 2048, 8), (40000, 2048, 11)])
+def test_lm_head_rows(N, K, M):
+    """Rows per pass over a large table: 2 (one-row kernel's form), 3 to 8 on the matrix cores, 11 = 8 + 3; partial last tiles of 64 rows, one and several tiles
+    per wave, 4 to 32 scale blocks (20: not a whole number of its groups of 16)."""
+    print(f"[lm_head rows] N={N} K={K} M={M}", flush=True)
+    rng = np.random.default_rng(N + M)
+    q = rng.integers(-127, 128, (N, K), dtype=np.int8)
+    s = (rng.random((N, K // 64), dtype=np.float32) + 0.5) * 1e-3
+    x = rng.standard_normal((M, K), dtype=np.float32) * np.exp(rng.standard_normal((M, 1))).astype(np.float32)
+    E = q35.Q8FTensor(dev(q), dev(s), q35.Q35_NK)
+    y = q35.q8_lm_head(dev(x), E)
+    for n0 in range(0, N, 1 << 15):
+        w = E.q[n0:n0 + (1 << 15)].double().view(-1, K // 64, 64) * E.scale[n0:n0 + (1 << 15)].double()[:, :, None]
+        ref = dev(x).double() @ w.view(-1, K).T.contiguous()
+        for m in range(M):
+            assert rel_l2(host(y[m, n0:n0 + (1 << 15)]), host(ref[m])) <= 1e-6, (m, n0)
+
+
+def test_lm_head_rows_infinity_as_one_row():
+    """A row with an infinity gives what the one-row kernel gives (infinite products, NaN where the
+    weight is 0); the other rows are not touched by it."""
+    N, K = 32768, 512
+    rng = np.random.default_rng(3)
+    E = q35.Q8FTensor(dev(rng.integers(-127, 128, (N, K), dtype=np.int8)),
+                      dev(rng.random((N, K // 64), dtype=np.float32) * 1e-2), q35.Q35_NK)
+    x = rng.standard_normal((3, K), dtype=np.float32)
+    x[1, 77] = np.inf
+    y = host(q35.q8_lm_head(dev(x), E))
+    np.testing.assert_array_equal(y[1], host(q35.q8_lm_head(dev(x[1:2]), E))[0])
+    for r in (0, 2):
+        assert rel_l2(y[r], host(q35.q8_lm_head(dev(x[r:r + 1]), E))[0]) <= 1e-6
