@@ -106,7 +106,7 @@ size_t q35_q8_gemv_ws_bytes(int32_t M, q35_q8f W);
 /* q35_q8_gemv without a workspace and without any allocation: no counterpart in the reference;
  * for callers that cannot allocate device memory (code under hipGraph capture, serving loops,
  * harnesses that forbid hipMalloc).  Same results as q35_q8_gemv (the same kernels).  The
- * Q35_KN / Q35_KN_TILED split-K scratch is a fixed 1 MiB + 64 KiB device array per GPU (held
+ * Q35_KN / Q35_KN_TILED split-K scratch is a fixed 9 MiB + 64 KiB device array per GPU (held
  * until the process ends), so min(M, 8) * N must be <= 131072 (else Q35_E_SHAPE); the panel and
  * NK layouts need no scratch.  Every call on one GPU shares that GPU's array, which each call
  * leaves zeroed: calls that overlap on one GPU (different streams, concurrent graph replays)

@@ -107,17 +107,17 @@ MvmSizes mvm_sizes(const q35_dims& d, int B) {
 }
 size_t mvm_layer_bytes(const q35_dims& d, int B) { return B >= kMvmMin ? mvm_sizes(d, B).bytes() : 0; }
 
-// One projection of a layer call over all of its rows, kMvmRows at a time: c carries the first
+// One projection of a layer call over all of its rows, g at a time: c carries the first
 // row's pointers and the partials.
-int mvm_rows(MvmCall c, int B, hipStream_t st) {
-  for (int b0 = 0; b0 < B; b0 += kMvmRows) {
-    c.M = std::min(kMvmRows, B - b0);
+int mvm_rows(MvmCall c, int B, hipStream_t st, int g = kMvmRows) {
+  for (int b0 = 0; b0 < B; b0 += g) {
+    c.M = std::min(g, B - b0);
     const int rc = mvm_launch(c, st);
     if (rc) return rc;
-    c.x += (size_t)kMvmRows * c.ldx;
-    c.y += (size_t)kMvmRows * c.ldy;
-    if (c.z) c.z += (size_t)kMvmRows * c.ldz;
-    if (c.bg) c.bg += (size_t)kMvmRows * 2 * c.aux_nh;
+    c.x += (size_t)g * c.ldx;
+    c.y += (size_t)g * c.ldy;
+    if (c.z) c.z += (size_t)g * c.ldz;
+    if (c.bg) c.bg += (size_t)g * 2 * c.aux_nh;
   }
   return Q35_OK;
 }
@@ -189,16 +189,27 @@ int q35_q8_gemv(const float* x, int32_t M, q35_q8f W, float* y, void* ws, size_t
   }
   if (W.layout != Q35_NK) {  // split-K with fixed-point sums; one launch per 8 rows
     const int K = W.rows, N = W.cols;
-    if (!ws || ws_bytes < q35_q8_gemv_ws_bytes(M, W)) return fail(Q35_E_WS, "q8_gemv: workspace too small");
+    const size_t accb = align256((size_t)std::min(M, 8) * N * sizeof(fx_t));
+    if (!ws || ws_bytes < kCounterBytes + accb) return fail(Q35_E_WS, "q8_gemv: workspace too small");
     fx_t* acc = reinterpret_cast<fx_t*>(ws_scratch(ws));
-    if (M >= kMvmGemvMin && mvm_ok(x, K, K) && mvm_ok(y, N, K)) {  // matrix cores, up to 32 rows per launch
+    // matrix cores, as many rows per launch as the workspace behind the accumulators has room for (the
+    // splits do not depend on the rows, so neither do a row's bits); less than 8: the one-row kernel
+    int g = 0;
+    // (sizes that q8_gemv_noalloc takes only where its fixed scratch has that room too: the two entry
+    // points give the same bits)
+    const bool fixed = (size_t)std::min(M, 8) * N * sizeof(fx_t) <= kNoAllocAccBytes;
+    if (M >= kMvmGemvMin && mvm_ok(x, K, K) && mvm_ok(y, N, K) &&
+        (!fixed || mvm_part_floats(std::min(M, 8), K, N, false) * sizeof(float) <= kNoAllocPartBytes))
+      for (g = kMvmRows; g >= 8 && mvm_part_floats(std::min(g, M), K, N, false) * sizeof(float) > ws_bytes - kCounterBytes - accb;)
+        g /= 2;
+    if (g >= 8) {
       MvmCall c;
       c.seg[0] = mvm_seg(W); c.nseg = 1; c.K = K; c.x = x; c.ldx = K; c.y = y; c.ldy = N;
-      c.part = reinterpret_cast<float*>(ws_scratch(ws) + align256((size_t)std::min(M, 8) * N * sizeof(fx_t)));
-      c.part_floats = mvm_part_floats(M, K, N, false);
+      c.part = reinterpret_cast<float*>(ws_scratch(ws) + accb);
+      c.part_floats = mvm_part_floats(std::min(g, M), K, N, false);
       c.clear = 1;  // (calls of other sizes place their zeroed sums there)
       c.err = ws_counters(ws) + kWsErrWord;
-      return mvm_rows(c, M, S(stream));
+      return mvm_rows(c, M, S(stream), g);
     }
     for (int m0 = 0; m0 < M; m0 += 8) {
       MvCall c;

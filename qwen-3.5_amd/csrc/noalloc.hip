@@ -1,7 +1,7 @@
 // q35_q8_gemv_noalloc: the Q8F matvec of q35_q8_gemv for callers that cannot allocate device
 // memory (code under hipGraph capture, serving loops, harnesses that forbid hipMalloc).  The
-// split-K path of the KN / KN_TILED layouts needs scratch (one completion counter per 256-column
-// tile and M x N fixed-point accumulators); here it lives in a file-scope device array of fixed
+// split-K paths of the KN / KN_TILED layouts need scratch (one completion counter per 256-column
+// tile and M x N fixed-point accumulators; from 4 rows on f32 partials); here it lives in a file-scope device array of fixed
 // size instead of a caller workspace.  The panel and NK layouts need no scratch and take the same
 // kernels as q35_q8_gemv.
 //
@@ -10,7 +10,8 @@
 // passed to kernels.  Every GPU holds its own copy until the process ends.  The counters and
 // accumulators must be zero when a call starts; the load-time image is zero, a fill kernel clears
 // the array once more on the first call on each device, and every call leaves both zero again
-// (the last block of each tile re-zeroes its accumulators and its counter).
+// (the last block of each tile re-zeroes its accumulators and its counter; the kernel that adds the
+// partials leaves zeros).
 #include "q35_host.h"
 
 #include <mutex>
@@ -19,8 +20,7 @@ namespace q35 {
 
 namespace {
 
-constexpr size_t kNoAllocAccBytes = (size_t)1 << 20;  // M * N <= 131072 fixed-point sums
-constexpr size_t kNoAllocBytes = kCounterBytes + kNoAllocAccBytes;
+constexpr size_t kNoAllocBytes = kCounterBytes + kNoAllocAccBytes + kNoAllocPartBytes;
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];

@@ -347,6 +347,9 @@ Q35_DEV void fx_add_chk(fx_t* p, float v, uint32_t* err) {
   if (fx_addable(v)) fx_add(p, v);
   else __hip_atomic_fetch_or((Q35_GLOBAL uint32_t*)err, kWsErrRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// q35_q8_gemv_noalloc's fixed scratch: a workspace of counters, 131072 fixed-point sums, and the split-K
+// partials of the multi-row path (8 rows of the widest call up to K = 8192)
+constexpr size_t kNoAllocAccBytes = (size_t)1 << 20, kNoAllocPartBytes = (size_t)8 << 20;
 inline char* ws_scratch(void* ws) { return static_cast<char*>(ws) + kCounterBytes; }
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 

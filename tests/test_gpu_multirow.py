@@ -144,3 +144,15 @@ def test_lm_head_rows_infinity_as_one_row():
     np.testing.assert_array_equal(y[1], host(q35.q8_lm_head(dev(x[1:2]), E))[0])
     for r in (0, 2):
         assert rel_l2(y[r], host(q35.q8_lm_head(dev(x[r:r + 1]), E))[0]) <= 1e-6
+
+
+@pytest.mark.parametrize("K,N,M", [(2048, 2048, 33), (6144, 2048, 20), (8192, 16384, 8), (8704, 16384, 8), (64, 64, 4)])
+def test_q8_gemv_noalloc_rows_same_bits(K, N, M):
+    """The allocation-free entry point takes the rows in smaller groups where its fixed scratch asks for
+    it, up to its largest (8704 x 16384 is past it: both entry points keep the one-row kernel), bit for bit."""
+    L = q35._lib
+    Wd = q8_dev(q8(480, K, N), q35.Q35_KN)
+    x = dev(normal(481, (M, K)))
+    y = torch.empty(M, N, device="cuda")
+    L.check(L.lib().q35_q8_gemv_noalloc(x.data_ptr(), M, Wd.desc(), y.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    np.testing.assert_array_equal(host(y), host(q35.q8_gemv(x, Wd)))
