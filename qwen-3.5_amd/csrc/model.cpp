@@ -376,14 +376,13 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
   for (int i = 0; i < seqs.n; ++i)
     if (seqs.p0[i] < 0 || (int64_t)seqs.p0[i] + seqs.row0[i + 1] - seqs.row0[i] > v.tmax)
       return fail(Q35_E_SHAPE, "prompt pass: positions past tmax");
-  // (from pageable memory: the copy has taken the table when the call returns)
-  if (seqs.n > 1) Q35_HIP_TRY(hipMemcpyAsync(m->pf_seqs, &seqs, sizeof(seqs), hipMemcpyHostToDevice, st));
   const PfArg sq = pf_arg(seqs, m->pf_seqs);
   const int T = sq.rows;
   const int H = d.hidden, F = d.ffn, nh = d.lin_heads, vdim = nh * d.lin_dv, key_dim = nh * d.lin_dk;
   const int conv_dim = 2 * key_dim + vdim, ah = d.attn_heads, kvh = d.kv_heads, hd = d.head_dim;
   const int LDY = m->pf_ldy;
   int rc;
+  if (seqs.n > 1 && (rc = store_seqs_launch(m->pf_seqs, seqs, st))) return rc;
   if ((rc = embed_seqs_launch(m->embed.q, m->embed.s, H, v.prompt, v.tmax, sq, m->pf_x, st))) return rc;
   // projections on the f16 matrix cores from the MB copies of the weights
   auto seg = [](const q35_model::Q8& w, const q35_model::Mb& mb, float* y, int ldy) {

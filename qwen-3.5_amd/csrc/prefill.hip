@@ -341,7 +341,7 @@ __global__ __launch_bounds__(kPP) void gdn_chunk_prep_kernel(const GdnPrefill a)
   __shared__ __align__(16) float Vs[kC][kLdq];
   __shared__ float U[kC][kC + 1];
   __shared__ float Tm[kC][kC + 1];
-  __shared__ float cum[kC], bet[kC], ecum[kC];
+  __shared__ float cum[kC], bet[kC], ecum[kC], edl[kC];  // e^cum, e^(cum_last - cum)
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int nchunk = a.sq.chunks, c = blockIdx.x % nchunk, h = blockIdx.x / nchunk;
@@ -389,14 +389,27 @@ __global__ __launch_bounds__(kPP) void gdn_chunk_prep_kernel(const GdnPrefill a)
   }
   for (int e = tid; e < kC * kC; e += kPP) U[e >> 6][e & 63] = 0.f;
   __syncthreads();
-  // l2norm of q (times dk^-1/2) and k rows
-  for (int r = wid; r < 2 * kC; r += kPP / 64) {
-    float* row = r < kC ? Qs[r] : Ks[r - kC];
-    const float v0 = row[lane], v1 = row[lane + 64];
-    const float rn = rsqrt_f(wave_sum(v0 * v0 + v1 * v1) + 1e-6f);
-    const float f = r < kC ? a.qscale : 1.0f;
-    row[lane] = (v0 * rn) * f;
-    row[lane + 64] = (v1 * rn) * f;
+  // l2norm of q (times dk^-1/2) and k rows, eight rows of a wave at a time (row by row, each waited for
+  // the previous one's LDS round trips)
+#pragma unroll
+  for (int r0 = 0; r0 < 2 * kC / (kPP / 64); r0 += 8) {
+    float v0[8], v1[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int r = wid + (r0 + u) * (kPP / 64);
+      const float* row = r < kC ? Qs[r] : Ks[r - kC];
+      v0[u] = row[lane];
+      v1[u] = row[lane + 64];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int r = wid + (r0 + u) * (kPP / 64);
+      float* row = r < kC ? Qs[r] : Ks[r - kC];
+      const float rn = rsqrt_f(wave_sum(v0[u] * v0[u] + v1[u] * v1[u]) + 1e-6f);
+      const float f = r < kC ? a.qscale : 1.0f;
+      row[lane] = (v0[u] * rn) * f;
+      row[lane + 64] = (v1[u] * rn) * f;
+    }
   }
   if (wid == 0) {  // cumulative decay inside the chunk (padded steps add 0): a wave scan
     float v = cum[lane];
@@ -407,6 +420,7 @@ __global__ __launch_bounds__(kPP) void gdn_chunk_prep_kernel(const GdnPrefill a)
     }
     cum[lane] = v;
     ecum[lane] = expf(v);
+    edl[lane] = expf(__shfl(v, kC - 1, 64) - v);
   }
   __syncthreads();
   // N = -(beta_i k_i.k_j) e^(cum_i - cum_j) for j < i; intra = (q_i.k_j) e^(cum_i - cum_j) for j <= i:
@@ -451,7 +465,7 @@ __global__ __launch_bounds__(kPP) void gdn_chunk_prep_kernel(const GdnPrefill a)
     const int l = 16 * lb + 4 * g, k = 16 * w + c16;
     float kv[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) kv[m] = Ks[l + m][k] * expf(cum[kC - 1] - cum[l + m]);
+    for (int m = 0; m < 4; ++m) kv[m] = Ks[l + m][k] * edl[l + m];
     *(float4*)(scr + kScrKd + scr_kd(l, k)) = make_float4(kv[0], kv[1], kv[2], kv[3]);
   }
   __syncthreads();
@@ -885,11 +899,22 @@ __global__ __launch_bounds__(kPT) void last_rows_kernel(const float* x, int ldx,
   if (threadIdx.x == 0) pos[slot] = s.p0 + s.T - 1;
 }
 
+__global__ void store_seqs_kernel(PfSeqs* p, const PfSeqs v) {
+  for (int i = threadIdx.x; i < (int)(sizeof(PfSeqs) / 4); i += blockDim.x)
+    reinterpret_cast<int32_t*>(p)[i] = reinterpret_cast<const int32_t*>(&v)[i];
+}
+
 __global__ void store_i32_kernel(int32_t* p, int32_t v) {
   if (threadIdx.x == 0) *p = v;
 }
 
 }  // namespace
+
+int store_seqs_launch(PfSeqs* p, const PfSeqs& v, hipStream_t st) {
+  hipLaunchKernelGGL(store_seqs_kernel, dim3(1), dim3(64), 0, st, p, v);
+  Q35_HIP_TRY(hipGetLastError());
+  return Q35_OK;
+}
 
 int store_i32_launch(int32_t* p, int32_t v, hipStream_t st) {
   hipLaunchKernelGGL(store_i32_kernel, dim3(1), dim3(64), 0, st, p, v);

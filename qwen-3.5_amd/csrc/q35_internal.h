@@ -749,6 +749,8 @@ Q35_DEV PfSeq pf_seq(const PfArg& a, int i) {
 }
 // Tokens per query tile of the prompt attention (16 query rows of one kv head).
 inline int32_t pf_attn_tile(int32_t nh, int32_t nkv) { return 16 / (nh / nkv); }
+// *p = v in stream order (from the kernel's arguments: no host copy has to outlive the call)
+int store_seqs_launch(PfSeqs* p, const PfSeqs& v, hipStream_t st);
 // x[t] = embedding of the prompt id at its sequence's position, prompt[slot * ldp + position]
 int embed_seqs_launch(const int8_t* q, const float* s, int D, const int32_t* prompt, int ldp, const PfArg& sq, float* x,
                       hipStream_t st);
