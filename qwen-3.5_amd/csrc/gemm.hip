@@ -22,6 +22,7 @@
 // logical tiles land on the same XCD (blocks are dispatched round-robin over the 8 XCDs), which
 // keeps a weight tile's re-reads inside one L2.
 #include "q35_internal.h"
+#include "split_k.h"
 
 #include <algorithm>
 
@@ -47,7 +48,8 @@ struct GArgs {
   int32_t nseg;
   const float* x;
   int32_t ldx, M, K, mtiles, accumulate, nblocks;
-  int32_t ksplit, kchunk, ncat;  // K splits of kchunk rows; partials part[split][M][ncat]
+  int32_t ksplit, ncat;  // K splits; partials part[split][M][ncat]
+  SplitK kst;            // their K steps (of kBK rows, MB path kHBK)
   float* part;
   float* amax;   // MB path: |x| maximum of each row [M]
   int32_t prep_rows;  // MB path: rows whose maximum the prep pass finds (M, or 0 when given)
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(kGT) void gemm_kernel(const GArgs a) {
     if (i < a.nseg && gt >= a.seg[i].tile0) sg = a.seg[i];
   const int n0 = (gt - sg.tile0) * BN, m0 = mt * BM;
   const int K = a.K;
-  const int kbeg = split * a.kchunk, kend = min(K, kbeg + a.kchunk);
+  const int kbeg = split_begin(a.kst, split) * kBK, kend = split_begin(a.kst, split + 1) * kBK;
 
   // ---- weight tile addressing
   // KN / KN_TILED: thread (r = tid % 32, c16 = tid / 32) loads row k0 + r, columns c16*16..+15.
@@ -374,7 +376,7 @@ __global__ __launch_bounds__(kGT, 2) void hgemm_kernel(const GArgs a) {
     if (i < a.nseg && gt >= a.seg[i].tile0) sg = a.seg[i];
   const int n0 = (gt - sg.tile0) * 128, m0 = mt * BM;
   const int K = a.K, nks = K >> 5;
-  const int kbeg = split * a.kchunk, kend = min(K, kbeg + a.kchunk);
+  const int kbeg = split_begin(a.kst, split) * kHBK, kend = split_begin(a.kst, split + 1) * kHBK;
   const int wm = w >> 1, wn = w & 1;
   const int cb = (n0 >> 6) + wn;  // the wave's column block within its segment
 
@@ -581,7 +583,7 @@ int launch_tile(const GemmCall& c, int ksplit, hipStream_t st) {
     ncat += s.N;
   }
   a.ksplit = ksplit;
-  a.kchunk = ((c.K / kBK + ksplit - 1) / ksplit) * kBK;
+  a.kst = split_k(c.K / kBK, ksplit);
   a.ncat = ncat;
   a.part = c.part;
   a.nblocks = tiles * ksplit * a.mtiles;
@@ -609,7 +611,7 @@ int launch_mb(const GemmCall& c, int ksplit, hipStream_t st) {
     ncat += s.N;
   }
   a.ksplit = ksplit;
-  a.kchunk = ((c.K / kHBK + ksplit - 1) / ksplit) * kHBK;
+  a.kst = split_k(c.K / kHBK, ksplit);
   a.ncat = ncat;
   a.part = c.part;
   a.nblocks = tiles * ksplit * a.mtiles;

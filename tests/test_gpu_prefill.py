@@ -174,6 +174,37 @@ def test_q8_gemm_mb_split_k_strided(M, K, N, accumulate):
     np.testing.assert_array_equal(y[:, :64], y0[:, :64])
 
 
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("K,N", [(3584, 1024), (2560, 2048), (2112, 128), (576, 256)])
+@pytest.mark.parametrize("M", [1, 37, 64, 65])
+def test_q8_gemm_mb_uneven_splits(M, K, N, accumulate):
+    """K steps of 64 that the splits do not divide (56, 40, 33 and 9 steps in up to 16 splits): every
+    split inside K, against float64."""
+    print(f"[gemm mb uneven] M={M} K={K} N={N} acc={accumulate}", flush=True)
+    W = q8(280 + K // 64 + N, K, N)
+    x, y0 = normal(281 + M, (M, K)), normal(282 + M, (M, N))
+    yd = dev(y0)
+    q35.q8_gemm(dev(x), q8_dev(W, q35.Q35_KN).mb(), yd, accumulate=accumulate)
+    ref = x.astype(np.float64) @ W.dequant() + (y0.astype(np.float64) if accumulate else 0.0)
+    assert rel_l2(host(yd), ref) <= 1e-5
+
+
+@pytest.mark.parametrize("layout", ["kn", "tiled", "nk"])
+def test_q8_gemm_split_k_uneven(layout):
+    """The same on the fp32 matrix cores: 18 and 66 steps of 32 in up to 4 splits."""
+    for M, K, N in [(37, 576, 128), (64, 2112, 256)]:
+        print(f"[gemm split uneven] M={M} K={K} N={N} {layout}", flush=True)
+        x = normal(291 + M, (M, K))
+        if layout == "nk":
+            E = q8(290 + K, N, K)
+            Wd, ref = q8_dev(E, q35.Q35_NK), x.astype(np.float64) @ E.dequant().T
+        else:
+            W = q8(290 + K, K, N)
+            Wd, ref = q8_dev(W, q35.Q35_KN), x.astype(np.float64) @ W.dequant()
+            Wd = Wd.tiled() if layout == "tiled" else Wd
+        assert rel_l2(host(q35.q8_gemm(dev(x), Wd, split_k=True)), ref) <= 1e-5
+
+
 # ---------------------------------------------------------------- Gated DeltaNet prompt path
 
 def test_gate_proj_prompt_input_rule():
