@@ -22,7 +22,6 @@
 // logical tiles land on the same XCD (blocks are dispatched round-robin over the 8 XCDs), which
 // keeps a weight tile's re-reads inside one L2.
 #include "q35_internal.h"
-#include "split_k.h"
 
 #include <algorithm>
 

@@ -280,9 +280,6 @@ int persistent(q35_model* m, int n, hipStream_t st, const int32_t* stop_ids = nu
 
 // ---- prompt path (TextForCausalLM::forward at seq_len > 1, model.rs:27-84,130-138)
 constexpr int kPrefillCap = 1024;  // tokens per pass; longer prompts run in passes
-// Rows up to which gate | up splits K and applies the SwiGLU in a second kernel: the fused epilogue
-// needs whole sums, and one 64-row tile is 96 blocks of the 2B shape's 12288 columns
-constexpr int kPrefillSplitGu = 64;
 
 SeqView model_view(q35_model* m) {
   SeqView v;
@@ -326,7 +323,7 @@ int ensure_prefill(q35_model* m, hipStream_t st) {
       (rc = dev_alloc_t(m, "prefill_bg", (size_t)cap * 2 * nh, &m->pf_bg)) ||
       (rc = dev_alloc_t(m, "prefill_q", (size_t)cap * ah * hd, &m->pf_q)) ||
       (rc = dev_alloc_t(m, "prefill_scratch", (size_t)nh * nchunk * kGdnScratchPerChunk, &m->pf_scr)) ||
-      (rc = dev_alloc_t(m, "prefill_partials", gemm_part_floats(cap, H), &m->pf_part)) ||
+      (rc = dev_alloc_t(m, "prefill_partials", prompt_part_floats(cap, H, F), &m->pf_part)) ||
       (rc = dev_alloc_t(m, "prefill_gemm_aux", gemm_aux_floats(cap), &m->pf_aux)) ||
       (rc = dev_alloc_t(m, "prefill_act_max", (size_t)cap, &m->pf_act_max)) ||
       (rc = dev_alloc_t(m, "prefill_seqs", 1, &m->pf_seqs)))
@@ -381,6 +378,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
   const int H = d.hidden, F = d.ffn, nh = d.lin_heads, vdim = nh * d.lin_dv, key_dim = nh * d.lin_dk;
   const int conv_dim = 2 * key_dim + vdim, ah = d.attn_heads, kvh = d.kv_heads, hd = d.head_dim;
   const int LDY = m->pf_ldy;
+  const size_t part_floats = prompt_part_floats(m->pf_cap, H, F);
   int rc;
   if (seqs.n > 1 && (rc = store_seqs_launch(m->pf_seqs, seqs, st))) return rc;
   if ((rc = embed_seqs_launch(m->embed.q, m->embed.s, H, v.prompt, v.tmax, sq, m->pf_x, st))) return rc;
@@ -405,7 +403,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
       g.x = m->pf_xn; g.ldx = H; g.M = T; g.K = H; g.nseg = 2;
       g.seg[0] = seg(L.qkv, W.qkv, m->pf_y, LDY);
       g.seg[1] = seg(L.z, W.z, m->pf_y + conv_dim, LDY);
-      g.part = m->pf_part; g.part_floats = gemm_part_floats(m->pf_cap, d.hidden); g.aux = m->pf_aux; g.amax = m->pf_aux;
+      g.part = m->pf_part; g.part_floats = part_floats; g.aux = m->pf_aux; g.amax = m->pf_aux;
       if ((rc = gemm_launch(g, st))) return rc;
       if ((rc = gate_prompt_launch(m->pf_xn, H, T, H, L.w_b, L.w_a, L.a_log, L.dt_bias, nh, m->pf_bg, st))) return rc;
       GdnPrefill gp;
@@ -421,7 +419,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
       o.x = m->pf_a; o.ldx = vdim; o.M = T; o.K = vdim; o.nseg = 1; o.accumulate = 1;
       o.seg[0] = seg(L.out, W.out, m->pf_x, H);
       o.defer_reduce = 1; o.ksplit_out = &pend;
-      o.part = m->pf_part; o.part_floats = gemm_part_floats(m->pf_cap, d.hidden); o.aux = m->pf_aux; o.amax = m->pf_aux;
+      o.part = m->pf_part; o.part_floats = part_floats; o.aux = m->pf_aux; o.amax = m->pf_aux;
       if ((rc = gemm_launch(o, st))) return rc;
     } else {
       const int qw = ah * hd * 2, kvw = kvh * hd;
@@ -430,7 +428,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
       g.seg[0] = seg(L.q, W.q, m->pf_y, LDY);
       g.seg[1] = seg(L.k, W.k, m->pf_y + qw, LDY);
       g.seg[2] = seg(L.v, W.v, m->pf_y + qw + kvw, LDY);
-      g.part = m->pf_part; g.part_floats = gemm_part_floats(m->pf_cap, d.hidden); g.aux = m->pf_aux; g.amax = m->pf_aux;
+      g.part = m->pf_part; g.part_floats = part_floats; g.aux = m->pf_aux; g.amax = m->pf_aux;
       if ((rc = gemm_launch(g, st))) return rc;
       AttnPrefill ap;
       ap.qg = m->pf_y; ap.ld_qg = LDY; ap.k = m->pf_y + qw; ap.v = m->pf_y + qw + kvw; ap.ld_kv = LDY;
@@ -443,7 +441,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
       o.x = m->pf_a; o.ldx = ah * hd; o.M = T; o.K = ah * hd; o.nseg = 1; o.accumulate = 1;
       o.seg[0] = seg(L.o, W.o, m->pf_x, H);
       o.defer_reduce = 1; o.ksplit_out = &pend;
-      o.part = m->pf_part; o.part_floats = gemm_part_floats(m->pf_cap, d.hidden); o.aux = m->pf_aux;
+      o.part = m->pf_part; o.part_floats = part_floats; o.aux = m->pf_aux;
       if ((rc = gemm_launch(o, st))) return rc;
     }
     if ((rc = rms_rows_launch(m->pf_x, H, T, H, L.post_norm, d.eps, m->pf_xn, H, st, m->pf_aux, pend > 1 ? m->pf_part : nullptr, pend,
@@ -460,7 +458,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
       g.seg[0] = seg(L.gate, W.gate, m->pf_y, LDY);
       g.seg[1] = seg(L.up, W.up, m->pf_y + F, LDY);
     }
-    g.part = m->pf_part; g.part_floats = gemm_part_floats(m->pf_cap, d.hidden); g.aux = m->pf_aux; g.amax = m->pf_aux;
+    g.part = m->pf_part; g.part_floats = part_floats; g.aux = m->pf_aux; g.amax = m->pf_aux;
     g.act = m->pf_a; g.ld_act = F; g.act_amax = m->pf_act_max;
     if ((rc = gemm_launch(g, st))) return rc;
     GemmCall dn;
@@ -468,7 +466,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
     dn.seg[0] = seg(L.down, W.down, m->pf_x, H);
     dn.defer_reduce = l + 1 < d.n_layers ? 1 : 0;  // (the lm_head reads the last residual row)
     dn.ksplit_out = &pend;
-    dn.part = m->pf_part; dn.part_floats = gemm_part_floats(m->pf_cap, d.hidden); dn.aux = m->pf_aux; dn.amax = m->pf_act_max;
+    dn.part = m->pf_part; dn.part_floats = part_floats; dn.aux = m->pf_aux; dn.amax = m->pf_act_max;
       if ((rc = gemm_launch(dn, st))) return rc;
   }
   return Q35_OK;

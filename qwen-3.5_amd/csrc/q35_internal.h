@@ -7,6 +7,7 @@
 #include <type_traits>
 #include "../../include/q35.h"
 #include "fx_range.h"
+#include "split_k.h"
 
 namespace q35 {
 
@@ -533,13 +534,6 @@ inline size_t gemm_aux_floats(int M) { return ((size_t)M + 63) / 64 * 64 + 64; }
 int gemm_launch(const GemmCall& c, hipStream_t st);
 // Tile shape and K splits the launcher picks for c (BM x BN, ksplit).
 int gemm_pick(const GemmCall& c, int* bm, int* bn, int* ksplit);
-// Partial floats that let gemm_launch consider up to kGemmMaxSplit K splits for M rows of N columns.
-// Few rows make few tiles, so the MB launches split further: one 64-row tile of a 2048-wide projection
-// is 16 blocks for 256 CUs.
-constexpr int kGemmMaxSplit = 4, kGemmMaxSplitMb = 16;
-inline size_t gemm_part_floats(int M, int64_t N) {
-  return (size_t)(M <= 64 ? 16 : (M <= 128 ? 8 : kGemmMaxSplit)) * M * N;
-}
 
 // ------------------------------------------------------------------ Q8F NK matvec / lm_head
 struct NkCall {

@@ -349,6 +349,23 @@ def test_model_prefill_states_match_token_by_token():
     b.close()
 
 
+@pytest.mark.parametrize("n_prompt", [1, 63, 64, 65])
+def test_model_prefill_wide_ffn(n_prompt):
+    """A model whose ffn is 8 times its hidden size, with prompts on both sides of the 64 rows up to
+    which gate | up goes through K-split partials: ids against the oracle."""
+    print(f"[model prefill wide ffn] prompt={n_prompt}", flush=True)
+    d = q35.make_dims(hidden=128, ffn=1024, vocab=4096, n_layers=4, lin_heads=4, attn_heads=4, kv_heads=2)
+    seed, tmax = 5, 150
+    prompt = np.random.default_rng(40 + n_prompt).integers(0, d.vocab, n_prompt).astype(np.int32)
+    rt, margins = oracle_model(d, seed, tmax).generate(prompt, 16)
+    m = q35.TextForCausalLM(d, seed=seed, tmax=tmax)
+    toks, _ = m.generate(prompt, 16, mode="stream", prefill=True)
+    m.check()
+    print("tokens", toks[:8], "min margin", margins.min(), flush=True)
+    np.testing.assert_array_equal(toks, rt)
+    m.close()
+
+
 def test_model_prefill_continuation_and_second_turn():
     """A prompt split over two prefill calls, then decoding, then a second prompt (a chat turn)
     through the prompt path: the ids equal the oracle's run of the same token sequence."""
