@@ -572,8 +572,8 @@ int q35_q8_gemm(const float* x, int32_t M, int32_t ldx, q35_q8f W, float* y, int
 size_t q35_q8_gemm_ws_bytes(int32_t M, q35_q8f W) {
   if (M < 1) return 0;
   const int N = W.layout == Q35_NK ? W.rows : W.cols;
-  const size_t aux = W.layout == Q35_KN_MB ? gemm_aux_floats(M) : 0;
-  return (aux + gemm_part_floats(M, N)) * sizeof(float);
+  if (W.layout == Q35_KN_MB) return (gemm_aux_floats(M) + mb_part_room(M, N, device_cus())) * sizeof(float);
+  return gemm_part_floats(M, N) * sizeof(float);
 }
 
 int q35_q8_gemm_ws(const float* x, int32_t M, int32_t ldx, q35_q8f W, float* y, int32_t ldy, int32_t accumulate,

@@ -24,6 +24,7 @@
 #include "q35_internal.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace q35 {
 namespace {
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(256) void gemm_swiglu_reduce_kernel(const GArgs a) 
 // written to LDS), weights and scales are loaded while the current step's MFMAs run.  Each lane
 // forms its own B operands (x row 16 i + c, 8 consecutive k) from the x tile and the column block's
 // scales in LDS.
-constexpr int kHBK = 64;          // K per main-loop step (two 32-row MB steps)
+constexpr int kHBK = kMbStepK;    // K per main-loop step (two 32-row MB steps)
 constexpr int kXLd = kHBK + 4;    // padded f32 row of the staged x tile (rows 4 banks apart)
 constexpr int kPrepS = 64;        // blocks of the scale-maximum pass (one wave's lanes)
 
@@ -557,17 +558,6 @@ __global__ __launch_bounds__(kGT, 2) void hgemm_kernel(const GArgs a) {
   }
 }
 
-int g_cus = 0;
-int device_cus() {
-  if (g_cus > 0) return g_cus;
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-    g_cus = n;
-  else
-    g_cus = 256;
-  return g_cus;
-}
-
 template <int BM, int BN>
 int launch_tile(const GemmCall& c, int ksplit, hipStream_t st) {
   GArgs a{};
@@ -645,36 +635,25 @@ int launch_mb(const GemmCall& c, int ksplit, hipStream_t st) {
 
 // MB path: 64 x 128 tiles (64-row tiles measured faster than 128-row ones at every prompt shape:
 // their 35 KB of LDS lets three or four blocks share a CU, so a launch spreads evenly over the
-// CUs) and the K split of least estimated time.  Measured at 512 rows: a block alone on a CU takes
-// ~1.09 us per 64-row K step, and a CU holding two or more blocks retires one block-step every
-// ~0.91 us; a split adds the reduction kernel (reads every split's partials, writes y: ~4 TB/s,
-// plus a launch).
-void gemm_pick_mb(const GemmCall& c, int* bm, int* ksplit) {
-  int64_t ncat = 0, tiles = 0;
-  for (int i = 0; i < c.nseg; ++i) {
-    ncat += c.seg[i].N;
-    tiles += c.seg[i].N / 128;
-  }
-  tiles *= (c.M + 63) / 64;
-  const int cus = device_cus();
-  double best = 1e300;
-  *bm = 64;
-  *ksplit = 1;
-  if (c.act && c.nseg == 1) return;  // (the SwiGLU epilogue needs whole sums)
-  for (int ks = 1; ks <= kGemmMaxSplitMb; ks *= 2) {
-    if (ks > 1 && (!c.part || c.part_floats < (size_t)ks * c.M * ncat || c.K / kHBK < 2 * ks)) break;
-    // past 4 splits only while half of them would leave half the CUs idle: the splits' reading back
-    // then costs more than the model's rate (2048 x 6144, 64 rows: 8 splits 23.3 us, 4 splits 22.4)
-    if (ks > kGemmMaxSplit && tiles * (ks / 2) > cus / 2) break;
-    const int steps = (c.K / kHBK + ks - 1) / ks;
-    const long long per_cu = (tiles * ks + cus - 1) / cus;
-    double cost = per_cu <= 1 ? steps * 1.09e-6 : (double)per_cu * steps * 0.91e-6;
-    if (ks > 1) cost += (double)c.M * ncat * (ks + 1) * 4.0 / 4e12 + (c.defer_reduce ? 0.0 : 3e-6);
-    if (cost < best * 0.97) { best = cost; *ksplit = ks; }
-  }
+// CUs) and the K split of least estimated time.
+int gemm_pick_mb(const GemmCall& c) {
+  if (c.act && c.nseg == 1) return 1;  // (the SwiGLU epilogue needs whole sums)
+  int64_t ncat = 0;
+  for (int i = 0; i < c.nseg; ++i) ncat += c.seg[i].N;
+  return mb_splits(c.M, ncat, c.K, device_cus(), c.defer_reduce != 0, c.part ? c.part_floats : 0);
 }
 
 }  // namespace
+
+int device_cus() {
+  static std::atomic<int> cache[64];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if ((n = cache[dev].load(std::memory_order_relaxed)) > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+  cache[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
 
 // Tile shape and K splits: the least estimated time.  A launch takes ceil(blocks / CUs) rounds,
 // each the block's MFMA work at the efficiency measured for its tile (128 x 128: 0.70 of peak per
@@ -731,9 +710,7 @@ int gemm_launch(const GemmCall& c, hipStream_t st) {
     if (c.act && (c.nseg > 2 || (c.nseg == 2 && (c.seg[0].N != c.seg[1].N || !c.part ||
                                                  c.part_floats < (size_t)c.M * 2 * c.seg[0].N)) || !c.act_amax || (c.ld_act % 4) != 0 || (reinterpret_cast<uintptr_t>(c.act) & 15)))
       return fail(Q35_E_ARG, "gemm: the SwiGLU output needs one segment (or gate, up and partials), row maxima and 16-byte aligned rows");
-    int bm = 64, ks = 1;
-    gemm_pick_mb(c, &bm, &ks);
-    return launch_mb<64>(c, ks, st);
+    return launch_mb<kMbTileM>(c, gemm_pick_mb(c), st);
   }
   if (c.M < 1 || c.K < kBK || (c.K % 64) != 0) return fail(Q35_E_SHAPE, "gemm: M >= 1 and K a multiple of 64 required");
   if ((c.ldx % 4) != 0 || (reinterpret_cast<uintptr_t>(c.x) & 15) != 0)

@@ -323,7 +323,7 @@ int ensure_prefill(q35_model* m, hipStream_t st) {
       (rc = dev_alloc_t(m, "prefill_bg", (size_t)cap * 2 * nh, &m->pf_bg)) ||
       (rc = dev_alloc_t(m, "prefill_q", (size_t)cap * ah * hd, &m->pf_q)) ||
       (rc = dev_alloc_t(m, "prefill_scratch", (size_t)nh * nchunk * kGdnScratchPerChunk, &m->pf_scr)) ||
-      (rc = dev_alloc_t(m, "prefill_partials", prompt_part_floats(cap, H, F), &m->pf_part)) ||
+      (rc = dev_alloc_t(m, "prefill_partials", prompt_part_floats(cap, H, F, device_cus()), &m->pf_part)) ||
       (rc = dev_alloc_t(m, "prefill_gemm_aux", gemm_aux_floats(cap), &m->pf_aux)) ||
       (rc = dev_alloc_t(m, "prefill_act_max", (size_t)cap, &m->pf_act_max)) ||
       (rc = dev_alloc_t(m, "prefill_seqs", 1, &m->pf_seqs)))
@@ -378,7 +378,7 @@ int prefill_pass(q35_model* m, const SeqView& v, const PfSeqs& seqs, hipStream_t
   const int H = d.hidden, F = d.ffn, nh = d.lin_heads, vdim = nh * d.lin_dv, key_dim = nh * d.lin_dk;
   const int conv_dim = 2 * key_dim + vdim, ah = d.attn_heads, kvh = d.kv_heads, hd = d.head_dim;
   const int LDY = m->pf_ldy;
-  const size_t part_floats = prompt_part_floats(m->pf_cap, H, F);
+  const size_t part_floats = prompt_part_floats(m->pf_cap, H, F, device_cus());
   int rc;
   if (seqs.n > 1 && (rc = store_seqs_launch(m->pf_seqs, seqs, st))) return rc;
   if ((rc = embed_seqs_launch(m->embed.q, m->embed.s, H, v.prompt, v.tmax, sq, m->pf_x, st))) return rc;

@@ -532,6 +532,8 @@ struct GemmCall {
 // Scratch floats of an MB launch: row maxima [M] and scale partial maxima [64], 64-aligned.
 inline size_t gemm_aux_floats(int M) { return ((size_t)M + 63) / 64 * 64 + 64; }
 int gemm_launch(const GemmCall& c, hipStream_t st);
+// Compute units of the current device (256 when there is none to ask)
+int device_cus();
 // Tile shape and K splits the launcher picks for c (BM x BN, ksplit).
 int gemm_pick(const GemmCall& c, int* bm, int* bn, int* ksplit);
 

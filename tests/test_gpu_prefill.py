@@ -189,6 +189,25 @@ def test_q8_gemm_mb_uneven_splits(M, K, N, accumulate):
     assert rel_l2(host(yd), ref) <= 1e-5
 
 
+@pytest.mark.parametrize("M", [64, 65, 128, 129, 300, 512])
+def test_q8_gemm_mb_same_bits_in_a_larger_workspace(M):
+    """The k / v projection with exactly the workspace it asks for, and with one that a larger call left
+    behind: the same bits."""
+    print(f"[gemm mb workspace] M={M}", flush=True)
+    K, N, L = 2048, 512, q35._lib
+    Wd = q8_dev(q8(285, K, N), q35.Q35_KN).mb()
+    x = dev(normal(286 + M, (M, K)))
+    ys = []
+    for extra in (0, 64 << 20):
+        nb = L.lib().q35_q8_gemm_ws_bytes(M, Wd.desc()) + extra
+        ws = torch.zeros(nb, dtype=torch.uint8, device="cuda")
+        y = torch.empty(M, N, device="cuda")
+        L.check(L.lib().q35_q8_gemm_ws(x.data_ptr(), M, K, Wd.desc(), y.data_ptr(), N, 0, ws.data_ptr(), nb,
+                                       torch.cuda.current_stream().cuda_stream))
+        ys.append(host(y))
+    np.testing.assert_array_equal(ys[0], ys[1])
+
+
 @pytest.mark.parametrize("layout", ["kn", "tiled", "nk"])
 def test_q8_gemm_split_k_uneven(layout):
     """The same on the fp32 matrix cores: 18 and 66 steps of 32 in up to 4 splits."""

@@ -6,7 +6,10 @@ A split that began at or past K read past the operands (its kernel loads the fir
 loop): with ceil(steps / splits) steps each, 56 steps in 16 splits left two of them.
 
 Room: the partials of a prompt pass hold a gate | up launch of up to 64 rows whatever the ratio of
-ffn to hidden (they were sized for the hidden width alone, and the launch was refused past 6 times it)."""
+ffn to hidden (they were sized for the hidden width alone, and the launch was refused past 6 times it).
+
+Same splits: a call takes the splits that unlimited room would give it with the room that is asked for
+its rows or for any larger call, so its bits do not depend on what a shared workspace grew to."""
 import os
 import subprocess
 
@@ -49,11 +52,43 @@ int main() {
     for (int hidden = 128; hidden <= 4096; hidden += 128)
       for (int ffn = 128; ffn <= 16 * hidden; ffn += 128) {
         const size_t need = (size_t)(cap < 64 ? cap : 64) * 2 * ffn;
-        if (q35::prompt_part_floats(cap, hidden, ffn) < need) {
+        if (q35::prompt_part_floats(cap, hidden, ffn, 256) < need) {
           std::printf("cap %d hidden %d ffn %d\n", cap, hidden, ffn);
           return 1;
         }
       }
+  return 0;
+}
+"""
+
+SAME = r"""
+#include <cstdio>
+#include "split_k.h"
+int main() {
+  long more = 0;
+  for (int cus : {256, 304, 64})
+    for (int N : {128, 512, 1024, 2048, 4096, 6144, 8192, 12288})
+      for (int K : {64, 576, 1024, 2048, 3584, 6144, 8192}) {
+        size_t room = 0;
+        for (int M = 1; M <= 1100; ++M) {
+          const size_t r = q35::mb_part_room(M, N, cus);
+          if (r < room) {
+            std::printf("room falls at M %d N %d\n", M, N);
+            return 1;
+          }
+          room = r;
+          for (int d = 0; d < 2; ++d) {
+            const int all = q35::mb_splits(M, N, K, cus, d, ~(size_t)0 >> 1);
+            more += all > 4;
+            if (q35::mb_splits(M, N, K, cus, d, r) != all || (all > 1 && (size_t)all * M * N > r)) {
+              std::printf("M %d N %d K %d cus %d: %d splits, asked room gives %d\n", M, N, K, cus, all,
+                          q35::mb_splits(M, N, K, cus, d, r));
+              return 1;
+            }
+          }
+        }
+      }
+  std::printf("%ld\n", more);
   return 0;
 }
 """
@@ -74,3 +109,7 @@ def test_every_split_lies_inside_k(tmp_path):
 
 def test_prompt_partials_hold_gate_up(tmp_path):
     run(tmp_path, ROOM)
+
+
+def test_asked_room_gives_the_same_splits(tmp_path):
+    assert int(run(tmp_path, SAME)) > 1000
