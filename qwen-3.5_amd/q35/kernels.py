@@ -155,7 +155,8 @@ def _gemv(fn, hidden_states, weights):
     rc = fn(x.data_ptr(), M, weights.desc(), y.data_ptr(), ws.data_ptr(), ws.numel(), _stream())
     if rc:
         L.check(rc)
-    return y if hidden_states.dim() == 2 else y.reshape(*hidden_states.shape[:-1], N)
+    # (rows that had to be regrouped to K wide do not fit their own shape: refused here)
+    return y if x is hidden_states else y.reshape(*hidden_states.shape[:-1], N)
 
 
 def q8_gemv(hidden_states, weights: Q8FTensor):

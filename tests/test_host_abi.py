@@ -134,3 +134,21 @@ def test_pack_kn_tiled_layout(K, N):
         np.testing.assert_array_equal(st[b // 4, :, b % 4], s[:, b])
     assert not qt[nt - 1, :, N - (nt - 1) * 256:].any()
     assert not st[nt - 1, :, N // 64 - (nt - 1) * 4:].any()
+
+
+def test_gemv_refuses_rows_of_another_width(monkeypatch):
+    """Rows whose width is not the weights' K are an error also where their elements would make whole
+    rows of K (4 x 1024 as 2 x 2048); every accepted shape keeps its leading dimensions.  The
+    library's call is a stand-in that computes nothing."""
+    from q35 import kernels
+
+    monkeypatch.setattr(kernels, "_stream", lambda: 0)
+    monkeypatch.setattr(kernels, "workspace", lambda n, *a: torch.zeros(16, dtype=torch.uint8))
+    K, N = 2048, 64
+    W = q35.Q8FTensor(torch.zeros(K, N, dtype=torch.int8), torch.zeros(K, 1), q35.Q35_KN)
+    for shape in [(K,), (3, K), (2, 1, K)]:
+        assert kernels._gemv(lambda *a: 0, torch.zeros(shape), W).shape == shape[:-1] + (N,)
+    assert kernels._gemv(lambda *a: 0, torch.zeros(3, 2 * K)[:, :K], W).shape == (3, N)
+    for shape in [(4, 1024), (2 * K,), (1, 2 * K), (2, 2, 1024)]:
+        with pytest.raises(RuntimeError):
+            kernels._gemv(lambda *a: 0, torch.zeros(shape), W)
