@@ -259,10 +259,10 @@ void launch_one(dim3 g, size_t lds, hipStream_t st, const NkArgs& a) {
   hipLaunchKernelGGL((nk_kernel<MR, CPW>), g, dim3(kThreads), lds, st, a);
 }
 
-// ---- 3 to 8 rows on the f16 matrix cores.  nk_kernel multiplies every weight by every row on the
+// ---- 3 to 8 rows on the bf16 matrix cores.  nk_kernel multiplies every weight by every row on the
 // vector ALUs, which bounds it from 2 rows on (248320 x 2048: 84 us at one row, 205 at 5, 364 at 8
 // with the final RMSNorm); here it is the table's stream again.  One block of 8 waves per CU stays for the
-// whole launch: its rows, split into three f16 values each (24 bits: q * x is exact before the f32
+// whole launch: its rows, split into three bf16 values each (24 bits: q * x is exact before the f32
 // accumulation; the block scales belong to the output rows here and are applied to each 64-k sum),
 // are staged in LDS once.  A wave walks tiles of 64 table rows: lane (g, c) = (lane / 16, lane % 16)
 // takes bytes 16 g .. 16 g + 15 of every 64-byte block of row 16 nt + c, the A operands of two products
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(kNmT, 1) void nkm_kernel(const NkArgs a) {
   extern __shared__ __align__(16) char nlds[];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
   const int K = a.K, nb = K >> 6, ldx = K + 8;
-  _Float16* xs = reinterpret_cast<_Float16*>(nlds);                                  // [3][8][ldx]
+  uint16_t* xs = reinterpret_cast<uint16_t*>(nlds);                                  // bf16 [3][8][ldx]
   float* sc = reinterpret_cast<float*>(nlds + (size_t)3 * kNmRows * ldx * 2) + w * 16 * kNmSld;  // [16][68]
   const int ntiles = (a.N + 63) / 64, stride = gridDim.x * kNmWaves;
   const int first = blockIdx.x * kNmWaves + w;
@@ -303,11 +303,10 @@ __global__ __launch_bounds__(kNmT, 1) void nkm_kernel(const NkArgs a) {
   };
 
   // wave w stages row w (rows past M repeat the last one; their outputs are dropped)
-  float inv;
   {
     const int m = min(w, a.M - 1);
     nf4 v[kNmKmax / 256], pw[kNmKmax / 256];
-    float ss = 0.f, mx = 0.f;
+    float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < kNmKmax / 256; ++i) {
       const int k = 256 * i + 4 * lane;
@@ -321,25 +320,17 @@ __global__ __launch_bounds__(kNmT, 1) void nkm_kernel(const NkArgs a) {
     for (int i = 0; i < kNmKmax / 256; ++i) ss += ((v[i][0] * v[i][0] + v[i][1] * v[i][1]) + v[i][2] * v[i][2]) + v[i][3] * v[i][3];
     const float r = a.pro == PRO_RMS ? rsqrt_f(wave_sum(ss) / (float)K + a.eps) : 1.0f;
 #pragma unroll
-    for (int i = 0; i < kNmKmax / 256; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (a.pro == PRO_RMS) v[i][j] = (v[i][j] * r) * (1.0f + pw[i][j]);
-        mx = fmaxf(mx, fabsf(v[i][j]));
-      }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    float f;
-    split_scale(mx, f, inv);
-    if (lane == 0) sc[0] = inv;
-#pragma unroll
     for (int i = 0; i < kNmKmax / 256; ++i) {
       const int k = 256 * i + 4 * lane;
       if (k >= K) break;
 #pragma unroll
       for (int j = 0; j < 4; j += 2) {
         uint32_t p[3];
-        const float y0 = v[i][j] * f, y1 = v[i][j + 1] * f;
+        float y0 = v[i][j], y1 = v[i][j + 1];
+        if (a.pro == PRO_RMS) {
+          y0 = (y0 * r) * (1.0f + pw[i][j]);
+          y1 = (y1 * r) * (1.0f + pw[i][j + 1]);
+        }
         split3(y0, y1, p[0], p[1], p[2]);
         // (an infinity has no remainder: its products are infinite, as in f32)
         if (fabsf(y0) == INFINITY) { p[1] &= 0xffff0000u; p[2] &= 0xffff0000u; }
@@ -349,8 +340,6 @@ __global__ __launch_bounds__(kNmT, 1) void nkm_kernel(const NkArgs a) {
       }
     }
   }
-  __syncthreads();
-  inv = (sc - w * 16 * kNmSld)[(c & 7) * 16 * kNmSld];  // of row c
   __syncthreads();
   if (total == 0) return;
 
@@ -373,20 +362,19 @@ __global__ __launch_bounds__(kNmT, 1) void nkm_kernel(const NkArgs a) {
           __builtin_amdgcn_wave_barrier();
         }
         // (a byte's place: k = 64 cb + 16 g + 8 h + j, products h = 0, 1)
-        q35_h8 b[3][2];
+        q35_b8 b[3][2];
 #pragma unroll
         for (int q = 0; q < 3; ++q)
 #pragma unroll
-          for (int h = 0; h < 2; ++h) b[q][h] = *(const q35_h8*)&xs[(q * kNmRows + (c & 7)) * ldx + 64 * cb + 16 * g + 8 * h];
+          for (int h = 0; h < 2; ++h) b[q][h] = *(const q35_b8*)&xs[(q * kNmRows + (c & 7)) * ldx + 64 * cb + 16 * g + 8 * h];
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) {
-          const q35_u32x4 wv = wr[d][nt] ^ 0x80808080u;  // int8 -> u = q + 128
-          const q35_h8 a0 = a8_from(wv[0], wv[1]), a1 = a8_from(wv[2], wv[3]);
+          const q35_b8 a0 = s8_from(wr[d][nt][0], wr[d][nt][1]), a1 = s8_from(wr[d][nt][2], wr[d][nt][3]);
           nf4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int q = 2; q >= 0; --q) {  // smallest parts first
-            t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b[q][0], t, 0, 0, 0);
-            t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, b[q][1], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[q][0], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[q][1], t, 0, 0, 0);
           }
           acc[nt] += t * *(const nf4*)&sc[(cb & 15) * kNmSld + 16 * nt + 4 * g];
         }
@@ -402,7 +390,7 @@ __global__ __launch_bounds__(kNmT, 1) void nkm_kernel(const NkArgs a) {
 #pragma unroll
               for (int i = 0; i < 4; ++i) {
                 const int n = 64 * ct + 16 * nt + 4 * g + i;
-                if (n < a.N) y[n] = acc[nt][i] * inv;
+                if (n < a.N) y[n] = acc[nt][i];
               }
           }
           ct += stride;

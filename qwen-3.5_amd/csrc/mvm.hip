@@ -1,22 +1,20 @@
-// Multi-row Q8F matvec (2..32 rows) on the f16 matrix cores for the reference's projection
+// Multi-row Q8F matvec (2..32 rows) on the bf16 matrix cores for the reference's projection
 // layouts (KN and its tile-major form): the layer calls of a batch of sequences and
 // multi-row q8_gemv (text_modules.rs:497-508, :855-893, :1003-1005; kernels.rs:53-92).
 //
 // What bounds it: the weight stream (each weight is read once for all rows).  The
 // one-row kernel's vector-ALU form multiplies every weight by every row, re-reads the weights
 // for each 8 rows and adds every column of every row with a 64-bit atomic; at 24 rows the MLP
-// spent 193 us on 38 MB of weights.  Here the products go to v_mfma_f32_16x16x32_f16 and the
+// spent 193 us on 38 MB of weights.  Here the products go to v_mfma_f32_16x16x32_bf16 and the
 // K splits leave plain f32 partials that a second kernel adds in split order.  Measured, 2B layer
 // calls: MLP at 24 rows 192.6 -> 33.6 us, DeltaNet at 9 rows 85.6 -> 27, the projections around the
 // attention of 16 rows 104 -> 24, q8_gemv 2048 x 6144 at 8 rows 35.0 -> 8.6.
 //
-// Arithmetic (f32-equivalent, as the other matrix-core paths): the int8 weight is exact in f16;
-// its block scale multiplies the input, y = x * s (f32), and y is carried whole, as three f16
-// values of y * 2^e (11 + 11 + 2 bits), with 2^e chosen from the largest |y| of the row over the
-// wave's K range: q * y is exact before the f32 accumulation.  The small values' products have an
+// Arithmetic (f32 products): the int8 weight is exact in bf16; its block scale multiplies the input,
+// y = x * s (f32), and y is carried whole, as three bf16 values (8 bits each): q * y is exact before
+// the f32 accumulation, whatever the range of the row.  The small values' products have an
 // accumulator of their own, added at the end (the matrix instruction's own additions do not always
-// round to nearest), so a single product comes out as the rounded f32 product.  (Two values, about
-// 22 bits, would save a third of the matrix instructions of a kernel that waits for memory.)
+// round to nearest), so a single product comes out as the rounded f32 product.
 //
 // Split: a wave owns one 64-column block x NS * 32 rows of K and issues all of its loads (a dword
 // of 4 columns per row and lane; its x rows; its scales) before the first use, so the launch's
@@ -32,7 +30,7 @@ namespace q35 {
 namespace {
 
 typedef q35_f32x4 f4;
-typedef q35_h8 h8;
+typedef q35_b8 b8;
 
 constexpr int kAuxRows = 128;  // K rows per gate-projection block
 constexpr int kAuxLd = 132;    // its padded f32 x row in LDS
@@ -55,20 +53,13 @@ struct MvmArgs {
 
 Q35_DEV f4 ld4(const float* p) { return *(const Q35_GLOBAL f4*)p; }
 
-// f16 operand of column byte nt of the 8 rows d[0..7]: bytes (row j, row j + 1) to the two halves,
-// then 0x6400 | (q + 128) = 1024 + 128 + q by one xor, minus 1152: exact.
+// bf16 operand of column byte NT of the 8 rows d[0..7].
 template <int NT>
-Q35_DEV h8 col8(const uint32_t (&d)[8]) {
-  constexpr uint32_t sel = 0x0c040c00u + NT * 0x00010001u;  // byte 0x0c selects 0x00
-  h8 r;
+Q35_DEV b8 col8(const uint32_t (&d)[8]) {
+  q35_u32x4 r;
 #pragma unroll
-  for (int j = 0; j < 8; j += 2) {
-    const uint32_t v = __builtin_amdgcn_perm(d[j + 1], d[j], sel) ^ 0x64806480u;
-    const q35_h2 p = __builtin_bit_cast(q35_h2, v) - q35_h2{(_Float16)1152.0f, (_Float16)1152.0f};
-    r[j] = p[0];
-    r[j + 1] = p[1];
-  }
-  return r;
+  for (int j = 0; j < 4; ++j) r[j] = bf_pair(s8_of<NT>(d[2 * j]), s8_of<NT>(d[2 * j + 1]));
+  return __builtin_bit_cast(b8, r);
 }
 
 // Gate projection (in_proj_b | in_proj_a, f32 [K][nh] each, kernels.rs:174-247): block ab sums
@@ -226,10 +217,7 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
     }
   }
 
-  // y = x * s in place, and each row's power of two
-  float f[MT], inv[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) f[mt] = 0.f;
+  // y = x * s in place
 #pragma unroll
   for (int st = 0; st < NS; ++st) {
     const bool in = k0 + 32 * st < a.K;
@@ -239,19 +227,8 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float y = in ? xv[st][mt][h][j] * s4[j] : 0.f;
-          xv[st][mt][h][j] = y;
-          f[mt] = fmaxf(f[mt], fabsf(y));
-        }
+        for (int j = 0; j < 4; ++j) xv[st][mt][h][j] = in ? xv[st][mt][h][j] * s4[j] : 0.f;
     }
-  }
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    float amax = f[mt];
-    amax = fmaxf(amax, __shfl_xor(amax, 16));
-    amax = fmaxf(amax, __shfl_xor(amax, 32));
-    split_scale(amax, f[mt], inv[mt]);
   }
 
   f4 acc[4][MT], accs[4][MT];
@@ -261,21 +238,20 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = accs[nt][mt] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int st = 0; st < NS; ++st) {
-    h8 b[3][MT];
+    b8 b[3][MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       uint32_t p[3][4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        split3(xv[st][mt][j >> 1][2 * (j & 1)] * f[mt], xv[st][mt][j >> 1][2 * (j & 1) + 1] * f[mt], p[2][j], p[1][j],
-               p[0][j]);
+        split3(xv[st][mt][j >> 1][2 * (j & 1)], xv[st][mt][j >> 1][2 * (j & 1) + 1], p[2][j], p[1][j], p[0][j]);
 #pragma unroll
-      for (int q = 0; q < 3; ++q) b[q][mt] = __builtin_bit_cast(h8, q35_u32x4{p[q][0], p[q][1], p[q][2], p[q][3]});
+      for (int q = 0; q < 3; ++q) b[q][mt] = __builtin_bit_cast(b8, q35_u32x4{p[q][0], p[q][1], p[q][2], p[q][3]});
     }
-    h8 aw[4];
+    b8 aw[4];
     if constexpr (LAY == LAY_SO) {
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) aw[nt] = a8_from(wv[st][2 * nt], wv[st][2 * nt + 1]);
+      for (int nt = 0; nt < 4; ++nt) aw[nt] = s8_from(wv[st][2 * nt] ^ 0x80808080u, wv[st][2 * nt + 1] ^ 0x80808080u);  // (bytes q + 128)
     } else {
       aw[0] = col8<0>(wv[st]);
       aw[1] = col8<1>(wv[st]);
@@ -286,14 +262,14 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
     for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        accs[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw[nt], b[0][mt], accs[nt][mt], 0, 0, 0);
-        acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw[nt], b[2][mt], acc[nt][mt], 0, 0, 0);
+        accs[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[nt], b[0][mt], accs[nt][mt], 0, 0, 0);
+        acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[nt], b[2][mt], acc[nt][mt], 0, 0, 0);
       }
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
-        accs[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw[nt], b[1][mt], accs[nt][mt], 0, 0, 0);
+        accs[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[nt], b[1][mt], accs[nt][mt], 0, 0, 0);
   }
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt)
@@ -301,15 +277,14 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] += accs[nt][mt];
 
   // lane holds column 16 g + 4 r + nt (stream order: 16 nt + 4 g + r) of row 16 mt + c in
-  // acc[nt][mt][r]; the waves' sums meet in LDS (2^-e undone first: it differs per wave) and are
-  // added in wave order
+  // acc[nt][mt][r]; the waves' sums meet in LDS and are added in wave order
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float* rr = &red[(w * 16 * MT + 16 * mt + c) * LD];
-      if constexpr (LAY == LAY_SO) *(f4*)(rr + 16 * r + 4 * g) = acc[r][mt] * inv[mt];
-      else *(f4*)(rr + 16 * g + 4 * r) = f4{acc[0][mt][r], acc[1][mt][r], acc[2][mt][r], acc[3][mt][r]} * inv[mt];
+      if constexpr (LAY == LAY_SO) *(f4*)(rr + 16 * r + 4 * g) = acc[r][mt];
+      else *(f4*)(rr + 16 * g + 4 * r) = f4{acc[0][mt][r], acc[1][mt][r], acc[2][mt][r], acc[3][mt][r]};
     }
   __syncthreads();
   const int ldp = 64 * a.ncb;

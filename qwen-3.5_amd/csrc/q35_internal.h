@@ -164,18 +164,34 @@ Q35_DEV void split2(float y0, float y1, uint32_t& hi, uint32_t& lo) {
   lo = __builtin_bit_cast(uint32_t, l);
 }
 
-// y -> three f16 values (packed conversions, rounding toward zero) whose sum is y, each remainder
-// exact in f32: 24 bits down to 2^-14 of the largest value (2^14 after scaling)
-Q35_DEV void split3(float y0, float y1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  const q35_hf2 h = __builtin_amdgcn_cvt_pkrtz(y0, y1);
-  const float r0 = y0 - (float)h[0], r1 = y1 - (float)h[1];
-  const q35_hf2 m = __builtin_amdgcn_cvt_pkrtz(r0, r1);
-  const q35_hf2 l = __builtin_amdgcn_cvt_pkrtz(r0 - (float)m[0], r1 - (float)m[1]);
-  hi = __builtin_bit_cast(uint32_t, h);
-  mid = __builtin_bit_cast(uint32_t, m);
-  lo = __builtin_bit_cast(uint32_t, l);
+// ---- the same with all of an f32 input's 24 bits, on the bf16 matrix cores
+// (v_mfma_f32_16x16x32_bf16): bf16 has the exponents of f32, so three values carry y whole whatever
+// the other inputs' magnitudes are (f16 parts under a common power of two hold all 24 bits only
+// down to 2^-14 of the largest), and 8-bit weights are exact in it too.
+typedef __bf16 q35_b8 __attribute__((ext_vector_type(8)));
+// The upper halves of two f32 values, one operand word
+Q35_DEV uint32_t bf_pair(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
-
+// y -> three bf16 values whose sum is y (8 bits each, rounding toward zero; the remainders are exact).
+// An infinity leaves NaN remainders.
+Q35_DEV void split3(float y0, float y1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+#pragma clang fp contract(off)  // (the remainder of the rounded y, not of a product behind it)
+  const float r0 = y0 - __uint_as_float(__float_as_uint(y0) & 0xffff0000u);
+  const float r1 = y1 - __uint_as_float(__float_as_uint(y1) & 0xffff0000u);
+  hi = bf_pair(y0, y1);
+  mid = bf_pair(r0, r1);
+  lo = bf_pair(r0 - __uint_as_float(__float_as_uint(r0) & 0xffff0000u),
+               r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u));
+}
+// Signed byte B of d (one conversion that selects and extends the byte)
+template <int B>
+Q35_DEV float s8_of(uint32_t d) { return (float)(int8_t)(d >> (8 * B)); }
+// The 8 signed weights of bytes 0..3 of da and 0..3 of db as a bf16 MFMA operand.
+Q35_DEV q35_b8 s8_from(uint32_t da, uint32_t db) {
+  return __builtin_bit_cast(q35_b8, q35_u32x4{bf_pair(s8_of<0>(da), s8_of<1>(da)), bf_pair(s8_of<2>(da), s8_of<3>(da)),
+                                              bf_pair(s8_of<0>(db), s8_of<1>(db)), bf_pair(s8_of<2>(db), s8_of<3>(db))});
+}
 
 Q35_DEV void fx_add(fx_t* p, float v) {
   __hip_atomic_fetch_add((Q35_GLOBAL unsigned long long*)p, (unsigned long long)to_fx(v), __ATOMIC_RELAXED,

@@ -62,6 +62,29 @@ def test_q8_gemv_rows_unaligned_input_and_magnitudes():
             assert rel_l2(y[m], ref[m] * float(mag[m])) <= 2e-6, m
 
 
+@pytest.mark.parametrize("layout", ["kn", "tiled", "nk"])
+@pytest.mark.parametrize("big", [2.0 ** 14, 2.0 ** 24, 2.0 ** 60])
+def test_rows_with_one_large_input_keep_f32_products(big, layout):
+    """One input per row many times the others, at a k whose weights are all 0: what is left are products
+    of ordinary size, as precise as without it (f32 sums as above; nk: the lm_head's rows)."""
+    print(f"[one large input] {big:.0e} {layout}", flush=True)
+    K, N, M = (512, 32768, 5) if layout == "nk" else (2048, 512, 5)
+    x = normal(435, (M, K))
+    x[:, 77] = big
+    if layout == "nk":
+        E = q8(436, N, K)
+        E.q[:, 77] = 0
+        y, ref = host(q35.q8_lm_head(dev(x), q8_dev(E, q35.Q35_NK))), x.astype(np.float64) @ E.dequant().T
+    else:
+        W = q8(436, K, N)
+        W.q[77] = 0
+        Wd = q8_dev(W, q35.Q35_KN)
+        y = host(q35.q8_gemv(dev(x), Wd.tiled() if layout == "tiled" else Wd))
+        ref = x.astype(np.float64) @ W.dequant()
+    for m in range(M):
+        assert rel_l2(y[m], ref[m]) <= 1e-6, m
+
+
 @pytest.mark.parametrize("B", [2, 33])
 def test_layers_in_row_groups(B):
     """MLP and attention over one row group and a second one (33 = 32 + 1 rows): each row as by itself."""
