@@ -25,6 +25,8 @@ namespace q35 {
 int batch_embed_f32_launch(const int8_t* q, const float* s, int D, const int32_t* token, const int32_t* prompt, int ldp,
                            const int32_t* plen, const int32_t* pos, float* h, fx_t* ss, fx_t* zero_ptr, int64_t zero_n,
                            uint32_t* err, int B, hipStream_t st);
+int rms_step_launch(float* h, int M, int K, const float* w, float eps, float* y, const float* part, int nsplit,
+                    uint32_t* err, hipStream_t st);
 int batch_argmax_groups(int V);
 int batch_argmax_launch(const float* logits, int V, int B, float* pv, int32_t* pi, int32_t* token, int32_t* pos,
                         int32_t* hist, int ldh, hipStream_t st);
@@ -204,7 +206,7 @@ int batch_layers_counted(q35_batch* bt, hipStream_t st) {
 
 // The layers' launches on the multi-row matvec (mvm.hip): every projection leaves its K splits as
 // plain partials; the next launch adds them, with the element-wise work between two projections in
-// it: the residual add and the RMSNorm (rms_rows), the SwiGLU, or the gates' activations.  The 2B step
+// it: the residual add and the RMSNorm (rms_step_kernel), the SwiGLU, or the gates' activations.  The 2B step
 // at 8 / 16 / 24 / 32 rows: 1433 / 1797 / 2853 / 3065 us with batch_layers_counted, which stages,
 // normalises and re-scales its input rows in every column block and hands K splits over through
 // returning atomics; 1378 / 1632 / 2119 / 2385 here.
@@ -227,11 +229,9 @@ int batch_layers_rows(q35_batch* bt, hipStream_t st) {
     int32_t ns = 0;
     c.nsplit_out = &ns;
     const int e = mvm_launch(c, st);
-    return e ? e : rms_rows_launch(bt->h + (size_t)r0 * H, H, c.M, H, w, d.eps, bt->xn + (size_t)r0 * H, H, st, nullptr,
-                                   bt->part, ns, (int64_t)c.M * H, H, nullptr, err);
+    return e ? e : rms_step_launch(bt->h + (size_t)r0 * H, c.M, H, w, d.eps, bt->xn + (size_t)r0 * H, bt->part, ns, err, st);
   };
-  if ((rc = rms_rows_launch(bt->h, H, B, H, m->layers[0].in_norm, d.eps, bt->xn, H, st, nullptr, nullptr, 0, 0, 0, nullptr, err)))
-    return rc;
+  if ((rc = rms_step_launch(bt->h, B, H, m->layers[0].in_norm, d.eps, bt->xn, nullptr, 0, err, st))) return rc;
   for (int l = 0; l < NL; ++l) {
     const q35_model::Layer& L = m->layers[l];
     const q35_model::MbLayer& W = m->mb[l];

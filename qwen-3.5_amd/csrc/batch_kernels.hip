@@ -1,9 +1,10 @@
 // Kernels of the batched decode step that the single-sequence kernels do not cover: the
-// per-sequence token selection + embedding into the fixed-point residual rows, and the
-// per-sequence greedy argmax over the logits rows (the reference's tie order), which advances
+// per-sequence token selection + embedding into the residual rows, the residual add and RMSNorm
+// between two projections of the multi-row matvec, and the per-sequence greedy argmax over the logits rows (the reference's tie order), which advances
 // each sequence's position and history.
 #include "q35_internal.h"
 
+#include <algorithm>
 #include <climits>
 
 namespace q35 {
@@ -49,6 +50,83 @@ __global__ __launch_bounds__(kBT) void batch_embed_f32_kernel(const int8_t* q, c
   if (threadIdx.x == 0) {
     if (!fx_addable(acc)) __hip_atomic_fetch_or((Q35_GLOBAL uint32_t*)err, kWsErrRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     ss[b] = fx_addable(acc) ? to_fx(acc) : 0;
+  }
+}
+
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+// x from lane (l + N) mod 16 of the 16-lane row, and the sum over a wave, of doubles (as row_ror and
+// wave_sum)
+template <int N>
+Q35_DEV double row_ror64(double x) {
+  const i32x2 u = __builtin_bit_cast(i32x2, x);
+  return __builtin_bit_cast(double, i32x2{__builtin_amdgcn_update_dpp(0, u[0], 0x120 + N, 0xf, 0xf, false),
+                                          __builtin_amdgcn_update_dpp(0, u[1], 0x120 + N, 0xf, 0xf, false)});
+}
+Q35_DEV double row_lane64(double x, int l) {
+  const i32x2 u = __builtin_bit_cast(i32x2, x);
+  return __builtin_bit_cast(double, i32x2{__builtin_amdgcn_readlane(u[0], l), __builtin_amdgcn_readlane(u[1], l)});
+}
+Q35_DEV double wave_sum64(double v) {
+  v += row_ror64<8>(v);
+  v += row_ror64<4>(v);
+  v += row_ror64<2>(v);
+  v += row_ror64<1>(v);
+  return (row_lane64(v, 0) + row_lane64(v, 16)) + (row_lane64(v, 32) + row_lane64(v, 48));
+}
+
+// Between two projections of the batched step: row m of h gets the residual projection's K splits
+// (part_0 + part_1 + ..., then h; NS of them, 0: none, -1: n, in groups of 16), and y the RMSNorm of the
+// new row, y = h * rsqrt(mean(h^2) + eps) * (1 + w).  The sums are 64-bit, as those of the step's
+// other launch sequence (fixed point) are.  A row whose sum of squares is not finite or reaches 2^31
+// raises kWsErrRange.
+// A block is a row, a thread 4 columns, so all loads of the row are one memory round trip, which with
+// the launch is what the kernel takes (16 rows of 2048, 12 / 8 splits: 4.7 / 4.5 us; with 256 threads and
+// f32 sums 5.0, the step at 16 rows 1635 -> 1613 us).
+constexpr int kRowMaxK = 4096;
+template <int NS>
+__global__ __launch_bounds__(kRowMaxK / 4) void rms_step_kernel(float* h, int K, const float* w, float eps, float* y,
+                                                                const float* part, int n, uint32_t* err) {
+  constexpr int G = NS > 0 ? NS : 16;
+  __shared__ double sh[kRowMaxK / 256];
+  const int tid = threadIdx.x, k = min(4 * tid, K - 4);  // (threads past the row repeat its end)
+  const bool in = 4 * tid < K;
+  float* hr = h + (int64_t)blockIdx.x * K + k;
+  q35_f32x4 v = *(const Q35_GLOBAL q35_f32x4*)hr;
+  const q35_f32x4 wv = *(const Q35_GLOBAL q35_f32x4*)(w + k);
+  if (NS != 0) {
+    const float* pr = part + (int64_t)blockIdx.x * K + k;
+    const int64_t stride = (int64_t)gridDim.x * K;
+    double t[4] = {0, 0, 0, 0};
+    for (int s0 = 0; s0 < (NS > 0 ? 1 : n); s0 += G) {
+      q35_f32x4 p[G];
+#pragma unroll
+      for (int u = 0; u < G; ++u)
+        p[u] = *(const Q35_GLOBAL q35_f32x4*)(pr + (NS > 0 ? u : min(s0 + u, n - 1)) * stride);
+#pragma unroll
+      for (int u = 0; u < G; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) t[j] += (NS > 0 || s0 + u < n) ? (double)p[u][j] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (float)(t[j] + v[j]);
+    if (in) *(Q35_GLOBAL q35_f32x4*)hr = v;
+  }
+  double ss = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ss += (double)v[j] * (double)v[j];
+  ss = wave_sum64(in ? ss : 0);
+  if ((tid & 63) == 0) sh[tid >> 6] = ss;
+  __syncthreads();
+  ss = 0;
+  for (int i = 0; i < (int)blockDim.x >> 6; ++i) ss += sh[i];
+  const float sf = (float)ss;
+  if (tid == 0 && !fx_addable(sf))
+    __hip_atomic_fetch_or((Q35_GLOBAL uint32_t*)err, kWsErrRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const float r = rsqrt_f(sf * rcp_f((float)K) + eps);
+  if (in) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (v[j] * r) * (1.0f + wv[j]);
+    *(Q35_GLOBAL q35_f32x4*)(y + (int64_t)blockIdx.x * K + k) = v;
   }
 }
 
@@ -121,6 +199,22 @@ int batch_embed_launch(const int8_t* q, const float* s, int D, const int32_t* to
                        const int32_t* plen, const int32_t* pos, fx_t* h, int B, hipStream_t st) {
   const int gx = std::min((D + kBT - 1) / kBT, 8);
   hipLaunchKernelGGL(batch_embed_kernel, dim3(gx, B), dim3(kBT), 0, st, q, s, D, token, prompt, ldp, plen, pos, h);
+  Q35_HIP_TRY(hipGetLastError());
+  return Q35_OK;
+}
+
+int rms_step_launch(float* h, int M, int K, const float* w, float eps, float* y, const float* part, int nsplit,
+                    uint32_t* err, hipStream_t st) {
+  if (M < 1 || K < 4 || K % 4 || K > kRowMaxK || nsplit < 0 || (nsplit > 0 && !part))
+    return fail(Q35_E_SHAPE, "rms_step: rows of up to 4096 columns, a multiple of 4");
+  using Fn = void (*)(float*, int, const float*, float, float*, const float*, int, uint32_t*);
+  static constexpr Fn fn[] = {rms_step_kernel<0>,  rms_step_kernel<1>,  rms_step_kernel<2>,  rms_step_kernel<3>,
+                              rms_step_kernel<4>,  rms_step_kernel<5>,  rms_step_kernel<6>,  rms_step_kernel<7>,
+                              rms_step_kernel<8>,  rms_step_kernel<9>,  rms_step_kernel<10>, rms_step_kernel<11>,
+                              rms_step_kernel<12>, rms_step_kernel<13>, rms_step_kernel<14>, rms_step_kernel<15>,
+                              rms_step_kernel<16>, rms_step_kernel<-1>};
+  hipLaunchKernelGGL(fn[std::min(nsplit, 17)], dim3(M), dim3((K / 4 + 63) / 64 * 64), 0, st, h, K, w, eps, y, part, nsplit,
+                     err);
   Q35_HIP_TRY(hipGetLastError());
   return Q35_OK;
 }

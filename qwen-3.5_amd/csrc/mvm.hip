@@ -298,28 +298,29 @@ __global__ __launch_bounds__(64 * NW) void mvm_kernel(const MvmArgs a) {
   }
 }
 
-// Adds the K splits in split order.  A partial that is not finite or whose magnitude reaches 2^31
-// is dropped and raises kWsErrRange, the contract of the one-row path's fixed-point sums.
-// clear: zeros are left in the partials' place.
+// Adds the K splits in split order, in 64 bits (the one-row path's sums are 64-bit fixed point).  A
+// partial that is not finite or whose magnitude reaches 2^31 is dropped and raises kWsErrRange, the
+// contract of those sums.  clear: zeros are left in the partials' place.  G splits are loaded at a time.
+template <int G>
 Q35_DEV f4 sum_splits(float* p, int nsplit, size_t stride, bool clear, bool& bad) {
-  f4 t = f4{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < nsplit; s += 8) {
-    f4 v[8];
+  double t[4] = {0, 0, 0, 0};
+  for (int s = 0; s < nsplit; s += G) {
+    f4 v[G];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = ld4(p + (size_t)min(s + u, nsplit - 1) * stride);
+    for (int u = 0; u < G; ++u) v[u] = ld4(p + (size_t)min(s + u, nsplit - 1) * stride);
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < G; ++u)
       if (s + u < nsplit) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const bool ok = fx_addable(v[u][j]);
           bad = bad || !ok;
-          t[j] += ok ? v[u][j] : 0.f;
+          t[j] += ok ? (double)v[u][j] : 0;
         }
         if (clear) *(Q35_GLOBAL f4*)(p + (size_t)(s + u) * stride) = f4{0.f, 0.f, 0.f, 0.f};
       }
   }
-  return t;
+  return f4{(float)t[0], (float)t[1], (float)t[2], (float)t[3]};
 }
 
 struct RedArgs {
@@ -332,6 +333,7 @@ struct RedArgs {
 };
 
 // One float4 of outputs per thread; the last block's threads finish the gates.
+template <int G>
 __global__ __launch_bounds__(256) void mvm_reduce_kernel(const RedArgs a) {
   const int nq = (a.swiglu ? a.N / 2 : a.N) / 4;
   const int64_t nout = (int64_t)a.M * nq;
@@ -342,14 +344,15 @@ __global__ __launch_bounds__(256) void mvm_reduce_kernel(const RedArgs a) {
     const int no = 2 * a.nh;
     for (int i = threadIdx.x; i < a.M * no; i += 256) {
       const int m = i / no, o = i - m * no, h = o < a.nh ? o : o - a.nh;
-      float v = 0.f;
+      double vs = 0;
       for (int s = 0; s < a.naux; s += 8) {
         float t[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) t[u] = ldg(a.aux + ((size_t)min(s + u, a.naux - 1) * a.M + m) * no + o);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v += s + u < a.naux ? t[u] : 0.f;
+        for (int u = 0; u < 8; ++u) vs += s + u < a.naux ? (double)t[u] : 0;
       }
+      float v = (float)vs;
       if (!fx_addable(v)) {
         bad = true;
         v = 0.f;
@@ -368,9 +371,9 @@ __global__ __launch_bounds__(256) void mvm_reduce_kernel(const RedArgs a) {
     if (i < nout) {
       const int m = (int)(i / nq), j = (int)(i - (int64_t)m * nq) * 4;
       float* p = a.part + (size_t)m * a.N + j;
-      f4 v = sum_splits(p, a.nsplit, stride, a.clear, bad);
+      f4 v = sum_splits<G>(p, a.nsplit, stride, a.clear, bad);
       if (a.swiglu) {
-        const f4 up = sum_splits(p + a.N / 2, a.nsplit, stride, a.clear, bad);
+        const f4 up = sum_splits<G>(p + a.N / 2, a.nsplit, stride, a.clear, bad);
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = up[r] * silu_f(v[r]);
       }
@@ -463,7 +466,8 @@ int mvm_launch(const MvmCall& c, hipStream_t st) {
   r.part = c.part; r.nsplit = p.nsplit; r.M = c.M; r.N = 64 * ncb; r.y = c.y; r.ldy = c.ldy;
   r.swiglu = c.swiglu; r.clear = c.clear; r.err = c.err;
   const int64_t nout = (int64_t)c.M * (c.swiglu ? r.N / 2 : r.N) / 4;
-  hipLaunchKernelGGL(mvm_reduce_kernel, dim3((unsigned)((nout + 255) / 256 + (r.naux ? 1 : 0))), dim3(256), 0, st, r);
+  const auto red = p.nsplit <= 2 ? mvm_reduce_kernel<2> : (p.nsplit <= 4 ? mvm_reduce_kernel<4> : mvm_reduce_kernel<8>);
+  hipLaunchKernelGGL(red, dim3((unsigned)((nout + 255) / 256 + (r.naux ? 1 : 0))), dim3(256), 0, st, r);
   Q35_HIP_TRY(hipGetLastError());
   return Q35_OK;
 }

@@ -75,8 +75,7 @@ Q35_DEV float4 sum_parts(const float* p, int64_t stride) {
 }
 __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K, const float* w, float eps,
                                                        float* y, int ldy, float* amax, const float* part,
-                                                       int nsplit, int64_t sstride, int ldp, float* clear,
-                                                       uint32_t* err) {
+                                                       int nsplit, int64_t sstride, int ldp, float* clear) {
   __shared__ float sh[4];
   const int m = blockIdx.x;
   if (clear && threadIdx.x == 0) clear[m] = 0.f;
@@ -100,12 +99,10 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
         const int k = 4 * (threadIdx.x + u * kPT);
         if (k < K) {
           float4 t;
-          switch (nsplit) {
-            case 1: t = sum_parts<1>(pr + k, sstride); break;
+          switch (nsplit) {  // (the GEMM splits by powers of two)
             case 2: t = sum_parts<2>(pr + k, sstride); break;
             case 4: t = sum_parts<4>(pr + k, sstride); break;
             case 8: t = sum_parts<8>(pr + k, sstride); break;
-            case 12: t = sum_parts<12>(pr + k, sstride); break;
             case 16: t = sum_parts<16>(pr + k, sstride); break;
             default:
               t = *(const float4*)(pr + k);
@@ -122,8 +119,6 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
 #pragma unroll
     for (int u = 0; u < kRmsHeld; ++u) ss += ((v[u].x * v[u].x + v[u].y * v[u].y) + v[u].z * v[u].z) + v[u].w * v[u].w;
     ss = block_sum256(ss, sh);
-    if (err && threadIdx.x == 0 && !fx_addable(ss))
-      __hip_atomic_fetch_or((Q35_GLOBAL uint32_t*)err, kWsErrRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const float r = rsqrt_f(ss * rcp_f((float)K) + eps);
 #pragma unroll
     for (int u = 0; u < kRmsHeld; ++u) {
@@ -149,8 +144,6 @@ __global__ __launch_bounds__(kPT) void rms_rows_kernel(float* x, int ldx, int K,
       ss += v * v;
     }
     ss = block_sum256(ss, sh);
-    if (err && threadIdx.x == 0 && !fx_addable(ss))
-      __hip_atomic_fetch_or((Q35_GLOBAL uint32_t*)err, kWsErrRange, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const float r = rsqrt_f(ss * rcp_f((float)K) + eps);
     for (int k = threadIdx.x; k < K; k += kPT) {
       const float v = (xr[k] * r) * (1.0f + w[k]);
@@ -938,11 +931,11 @@ int last_rows_launch(const float* x, int ldx, int D, const PfArg& sq, float* h, 
 
 int rms_rows_launch(float* x, int ldx, int M, int K, const float* w, float eps, float* y, int ldy,
                     hipStream_t st, float* amax, const float* part, int nsplit, int64_t sstride, int ldp,
-                    float* clear, uint32_t* err) {
+                    float* clear) {
   if (M < 1) return Q35_OK;
   if (part && nsplit < 1) return fail(Q35_E_ARG, "rms_rows: no splits in the partials");
   hipLaunchKernelGGL(rms_rows_kernel, dim3(M), dim3(kPT), 0, st, x, ldx, K, w, eps, y, ldy, amax,
-                     part, nsplit, sstride, ldp, clear, err);
+                     part, nsplit, sstride, ldp, clear);
   Q35_HIP_TRY(hipGetLastError());
   return Q35_OK;
 }

@@ -773,11 +773,10 @@ int store_i32_launch(int32_t* p, int32_t v, hipStream_t st);
 // y[m] = RMSNorm(x[m]) * (1 + w) for M rows of K
 // y = RMSNorm(x) (1 + w) per row; amax (optional): each row's max |y|.  part (optional):
 // nsplit K-split partial sums of a deferred GEMM that accumulates into x: x = ((part_0 + part_1) + ...)
-// + x is formed and written back to x first (split s, row m at part + s * sstride + m * ldp).  err
-// (optional): receives kWsErrRange when a row's sum of squares is not finite or >= 2^31.
+// + x is formed and written back to x first (split s, row m at part + s * sstride + m * ldp).
 int rms_rows_launch(float* x, int ldx, int M, int K, const float* w, float eps, float* y, int ldy,
                     hipStream_t st, float* amax = nullptr, const float* part = nullptr, int nsplit = 1,
-                    int64_t sstride = 0, int ldp = 0, float* clear = nullptr, uint32_t* err = nullptr);
+                    int64_t sstride = 0, int ldp = 0, float* clear = nullptr);
 // [beta | g] rows of a prompt (x [T][ldx], softplus identity branch when its input exceeds 20)
 int gate_prompt_launch(const float* x, int ldx, int T, int K, const float* wb, const float* wa, const float* alog,
                        const float* dtb, int nh, float* out, hipStream_t st);

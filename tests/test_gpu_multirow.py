@@ -85,6 +85,26 @@ def test_rows_with_one_large_input_keep_f32_products(big, layout):
         assert rel_l2(y[m], ref[m]) <= 1e-6, m
 
 
+@pytest.mark.parametrize("layout", ["kn", "tiled"])
+@pytest.mark.parametrize("N,M", [(512, 4), (4096, 5), (6144, 17)])
+def test_k_splits_are_added_in_64_bits(N, M, layout):
+    """2^24 from the first rows of K, 1 from the middle and -2^24 from the last, each exact in its own
+    split: the sum is 1 as with one row, where 32-bit sums leave 0 (the widths take 16, 8 and 4 splits)."""
+    print(f"[64-bit splits] N={N} M={M} {layout}", flush=True)
+    K = 2048
+    W = q8(437, K, N)
+    W.q[:] = 0
+    W.s[:] = 1.0
+    W.q[0] = W.q[K - 1] = 64
+    W.q[K // 2] = 1
+    x = np.zeros((M, K), np.float32)
+    x[:, 0], x[:, K // 2], x[:, K - 1] = 2.0 ** 18, 1.0, -2.0 ** 18
+    Wd = q8_dev(W, q35.Q35_KN)
+    Wd = Wd.tiled() if layout == "tiled" else Wd
+    for rows in (M, 1):
+        np.testing.assert_array_equal(host(q35.q8_gemv(dev(x[:rows]), Wd)), 1.0)
+
+
 @pytest.mark.parametrize("B", [2, 33])
 def test_layers_in_row_groups(B):
     """MLP and attention over one row group and a second one (33 = 32 + 1 rows): each row as by itself."""
