@@ -269,6 +269,7 @@ void launch_one(dim3 g, size_t lds, hipStream_t st, const NkArgs& a) {
 // (k order permuted alike on both operands), four blocks ahead, across the tile's end.  The 64
 // rows' scales of 16 blocks pass through the wave's own LDS, loaded one group ahead.
 // 120 us at 2, 3 and 5 rows, 123 at 8 (4.4 TB/s), so 2 rows stay with nk_kernel.
+// (K up to 2048: the rows' planes take 96 KB of LDS there, and the prologue holds a row in registers)
 constexpr int kNmRows = 8, kNmWaves = 8, kNmT = 64 * kNmWaves, kNmKmax = 2048;
 constexpr int kNmSld = 68;  // padded row of 64 staged scales
 typedef q35_f32x4 nf4;
@@ -410,15 +411,6 @@ bool nkm_ok(const NkCall& c) {
          (c.pro != PRO_RMS || (reinterpret_cast<uintptr_t>(c.pw) & 15) == 0) && nkm_lds(c.K) <= lds_per_block();
 }
 
-int nkm_cus() {
-  static int n = 0;
-  if (!n) {
-    int dev = 0, v = 0;
-    n = (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) ? v : 256;
-  }
-  return n;
-}
-
 template <int MR>
 void launch_mr(int cpw, dim3 g, size_t lds, hipStream_t st, const NkArgs& a) {
   if (cpw == 1) launch_one<MR, 1>(g, lds, st, a);
@@ -471,7 +463,7 @@ int nk_launch(const NkCall& c, void* ws, size_t ws_bytes, hipStream_t st) {
   if (nkm_ok(c)) {
     const size_t nl = nkm_lds(c.K);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(nkm_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)nl);
-    hipLaunchKernelGGL(nkm_kernel, dim3(std::min(nkm_cus(), (c.N + 64 * kNmWaves - 1) / (64 * kNmWaves))), dim3(kNmT), nl, st, a);
+    hipLaunchKernelGGL(nkm_kernel, dim3(std::min(device_cus(), (c.N + 64 * kNmWaves - 1) / (64 * kNmWaves))), dim3(kNmT), nl, st, a);
     Q35_HIP_TRY(hipGetLastError());
     return Q35_OK;
   }
