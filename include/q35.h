@@ -94,12 +94,18 @@ q35_dims q35_dims_qwen35_2b(void);
 
 /* y[M][N] = x[M][K] @ dequant(W).  W.layout selects KN (reference projections), its tiled or
  * panel re-layouts, or NK.  Full-K semantics (every input row is summed).  M in [1, 64]; K, N
- * multiples of 64.  One kernel launch per 8 rows of x (Q35_KN_PANEL needs no workspace: ws may
- * be NULL).  Replaces q8_gemv (src/kernels.rs:681-688, kernel :53-92). */
+ * multiples of 64.  Q35_KN / Q35_KN_TILED: up to 3 rows, one launch; from 4 rows on (x and y 16-byte
+ * aligned, else one launch per 8 rows as below 4) two launches per group of up to 32 rows, the products
+ * on the matrix cores and the sum of the K splits.  Both sum f32 products; they differ in rounding.  A
+ * workspace smaller than the *_ws_bytes() of M rows takes them in smaller groups, with the same
+ * bits, and below the room for 8 rows' splits keeps the first form, whose bits differ.
+ * Q35_KN_PANEL: one launch per 8 rows, no workspace (ws may be NULL); Q35_NK: one per 8 rows at most.
+ * Replaces q8_gemv (src/kernels.rs:681-688, kernel :53-92). */
 int q35_q8_gemv(const float* x, int32_t M, q35_q8f W, float* y, void* ws, size_t ws_bytes, void* stream);
 
 /* Same contract; replaces q8_gemv_partial_sum (src/kernels.rs:690-700, impl :495-537, kernels
- * :103-165) whose split-K reduction is done here deterministically inside one launch. */
+ * :103-165) whose split-K reduction is done here deterministically, inside the launch (up to 3 rows)
+ * or by a second one. */
 int q35_q8_gemv_partial_sum(const float* x, int32_t M, q35_q8f W, float* y, void* ws, size_t ws_bytes, void* stream);
 size_t q35_q8_gemv_ws_bytes(int32_t M, q35_q8f W);
 

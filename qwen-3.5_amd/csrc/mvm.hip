@@ -387,7 +387,8 @@ __global__ __launch_bounds__(256) void mvm_reduce_kernel(const RedArgs a) {
 struct MvmPlan { int ns, nw, nsplit; };
 
 // Rows of K per wave (64 or 128) and waves per block (2 or 4): the most rows per block that still
-// give about two blocks per CU, so that few partials are written while every CU streams.
+// give 384 blocks, one and a half per CU, so that few partials are written while every CU streams.  (A
+// number and not the device's: the plan fixes the partials' size and a call's bits.)
 MvmPlan mvm_plan(int ncb, int K, bool gated) {
   const int cand[3][2] = {{4, 4}, {4, 2}, {2, 2}};
   MvmPlan p{4, 2, 1};

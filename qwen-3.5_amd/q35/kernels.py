@@ -35,10 +35,6 @@ def _stream():
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
-def ctypes_stream(s):
-    return s.cuda_stream
-
-
 def workspace(nbytes, device=None, key="default"):
     """Zero-filled scratch for one kind of entry point on the current stream.  Each call leaves
     its completion counters and fixed-point accumulators zero again, so a buffer serves every
