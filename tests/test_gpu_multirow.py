@@ -1,7 +1,8 @@
-"""The multi-row matrix-core matvec (q8_gemv from 2 rows, layer calls from 2 sequences) against
+"""The multi-row matrix-core matvec (q8_gemv from 4 rows, layer calls from 2 sequences) against
 float64: edges of its row tiles (16, 32, 33 rows), of its column blocks and tiles (64, 320: a partial
-256-column tile), of its K ranges (64: one short wave; 160: a range that ends inside a block), both
-layouts, and one workspace shared by calls of different sizes and row counts.
+256-column tile), of its K ranges (64: one short wave; 160: a range that ends inside a block; 2112: a
+wave that lies past K), both layouts, and one workspace shared by calls of different sizes and row
+counts.
 
 Bound: the products are exact and the sums f32 over K <= 6144 (a few 2^-24 per partial sum, random
 signs: seen 1e-7 to 3e-7); 2e-6 is taken."""
@@ -17,7 +18,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("layout", ["kn", "tiled"])
-@pytest.mark.parametrize("K,N,M", [(64, 64, 2), (160, 320, 3), (2048, 512, 16), (2048, 6144, 17), (6144, 2048, 32),
+@pytest.mark.parametrize("K,N,M", [(64, 64, 4), (160, 320, 5), (2112, 320, 6), (2048, 512, 16), (2048, 6144, 17), (6144, 2048, 32),
                                    (2048, 2048, 33), (96, 192, 64)])
 def test_q8_gemv_rows(K, N, M, layout):
     print(f"[gemv rows] K={K} N={N} M={M} {layout}", flush=True)

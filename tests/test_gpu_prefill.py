@@ -157,9 +157,10 @@ def test_q8_gemm_mb_row_magnitudes_and_zero_rows():
 
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("K,N", [(2048, 2048), (6144, 2048), (4096, 2048)])
-@pytest.mark.parametrize("M", [130, 512])
+@pytest.mark.parametrize("M", [1, 37, 64, 65, 128, 130, 512])
 def test_q8_gemm_mb_split_k_strided(M, K, N, accumulate):
-    """The MB path's split-K launches and the residual add into a strided y slice."""
+    """The MB path's split-K launches (up to 16 splits for one row tile, 8 for two, 4 above) and the
+    residual add into a strided y slice."""
     print(f"[gemm mb split] M={M} K={K} N={N} acc={accumulate}", flush=True)
     W = q8(270 + K // 64 + N, K, N)
     xf = normal(271 + M, (M, K + 64))
@@ -276,11 +277,14 @@ def test_gated_delta_rule_prefill_matches_recurrent_steps(T, warm):
 
 # ---------------------------------------------------------------- attention prompt path
 
-@pytest.mark.parametrize("T,p0", [(1, 0), (17, 0), (100, 0), (33, 40), (64, 0), (130, 300), (5, 500)])
+@pytest.mark.parametrize("T,p0", [(1, 0), (17, 0), (100, 0), (33, 40), (64, 0), (130, 300), (5, 500), (256, 0),
+                                  (257, 0), (300, 77), (517, 40)])
 def test_attention_core_prefill(T, p0):
     """C3 head layout (8 q heads, 2 kv heads, 256 dims, RoPE on 64, theta 1e7): rows at
     positions p0..p0+T-1 attend causally to the cache rows 0..p0+t.  The cases cover one and many
-    16-key tiles per wave, a ragged last tile and a long cached context before a short prompt."""
+    16-key tiles per wave, a ragged last tile, a long cached context before a short prompt, and both
+    sides of the 128 blocks (256 rows here) up to which a block has 8 waves, past them with a cached
+    context too."""
     print(f"[attention prefill] T={T} p0={p0}", flush=True)
     d = q35.dims_2b()
     nh, nkv, hd = d.attn_heads, d.kv_heads, d.head_dim
@@ -366,6 +370,28 @@ def test_model_prefill_states_match_token_by_token():
     assert a.position() == b.position() == 150
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("n_prompt", [1, 63, 64, 65])
+def test_prompt_gate_up_rows_and_their_maxima(n_prompt):
+    """Both forms of a prompt's gate | up (up to 64 rows through K-split partials, above in the GEMM's
+    epilogue): the last layer's rows up * silu(gate) against float64 of the rows it read, and the row
+    maxima that the down projection scales by, exactly those of the rows."""
+    print(f"[prompt gate up] prompt={n_prompt}", flush=True)
+    d, seed = hybrid_dims(), 3
+    H, F, l = d.hidden, d.ffn, d.n_layers - 1
+    m = q35.TextForCausalLM(d, seed=seed, tmax=128)
+    m.prefill(np.random.default_rng(50 + n_prompt).integers(0, d.vocab, n_prompt).astype(np.int32))
+    x = m.tensor("prefill_xn", np.float32).reshape(-1, H)[:n_prompt].astype(np.float64)
+    act = m.tensor("prefill_a", np.float32)[:n_prompt * F].reshape(n_prompt, F)
+    w = {n: O.quantize(q35.synth_model_tensor(d, seed, f"layers.{l}.mlp.{n}", H * F).reshape(H, F)).dequant()
+         for n in ("gate_proj", "up_proj")}
+    gate = x @ w["gate_proj"]
+    ref = (x @ w["up_proj"]) * gate / (1 + np.exp(-gate))
+    for r in range(n_prompt):
+        assert rel_l2(act[r], ref[r]) <= 1e-5, r
+    np.testing.assert_array_equal(m.tensor("prefill_act_max", np.float32)[:n_prompt], np.abs(act).max(axis=1))
+    m.close()
 
 
 @pytest.mark.parametrize("n_prompt", [1, 63, 64, 65])
