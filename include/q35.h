@@ -259,7 +259,7 @@ size_t q35_q8_gemm_ws_bytes(int32_t M, q35_q8f W);
 int q35_q8_gemm_ws(const float* x, int32_t M, int32_t ldx, q35_q8f W, float* y, int32_t ldy, int32_t accumulate,
                    void* ws, size_t ws_bytes, void* stream);
 
-/* The batched decode's projection (the kernel behind q35_batch_*) on its own: y[m][n] (+)=
+/* A projection of batch rows (the kernel behind q35_batch_* of up to 4 rows) on its own: y[m][n] (+)=
  * in[m][:] . dequant(W)[:, n] for M <= 32 rows on the f16 matrix cores (x * scale as f16 hi + lo,
  * about 22 significant bits; f32 accumulation), W in Q35_KN_MB (rows = K, cols = N, both multiples
  * of 128).  The prologue forms in[m] from the x row (ldx floats apart, 16-byte aligned):

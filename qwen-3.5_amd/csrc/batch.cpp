@@ -99,8 +99,7 @@ void bdestroy(q35_batch* b) {
 hipStream_t bpick(q35_batch* b, void* s) { return s ? static_cast<hipStream_t>(s) : b->own_stream; }
 
 // The layers' launches with the residual adds and norm statistics inside the projections
-// (mb_launch), for up to 4 rows and for
-// value heads other than 128 wide.
+// (mb_launch), for up to 4 rows and for value heads other than 128 wide.
 int batch_layers_counted(q35_batch* bt, hipStream_t st) {
   const q35_model* m = bt->m;
   const q35_dims& d = m->d;
@@ -209,7 +208,7 @@ int batch_layers_counted(q35_batch* bt, hipStream_t st) {
 // it: the residual add and the RMSNorm (rms_step_kernel), the SwiGLU, or the gates' activations.  The 2B step
 // at 8 / 16 / 24 / 32 rows: 1433 / 1797 / 2853 / 3065 us with batch_layers_counted, which stages,
 // normalises and re-scales its input rows in every column block and hands K splits over through
-// returning atomics; 1378 / 1632 / 2119 / 2385 here.
+// returning atomics; 1370 / 1613 / 2086 / 2349 here.
 int batch_layers_rows(q35_batch* bt, hipStream_t st) {
   const q35_model* m = bt->m;
   const q35_dims& d = m->d;

@@ -268,7 +268,7 @@ void launch_one(dim3 g, size_t lds, hipStream_t st, const NkArgs& a) {
 // takes bytes 16 g .. 16 g + 15 of every 64-byte block of row 16 nt + c, the A operands of two products
 // (k order permuted alike on both operands), four blocks ahead, across the tile's end.  The 64
 // rows' scales of 16 blocks pass through the wave's own LDS, loaded one group ahead.
-// 120 us at 2, 3 and 5 rows, 123 at 8 (4.4 TB/s), so 2 rows stay with nk_kernel.
+// 117 us at 3, 118 at 5, 120 at 8 rows (4.5 TB/s); 2 rows took 110 us in nk_kernel and 120 here, and stay there.
 // (K up to 2048: the rows' planes take 96 KB of LDS there, and the prologue holds a row in registers)
 constexpr int kNmRows = 8, kNmWaves = 8, kNmT = 64 * kNmWaves, kNmKmax = 2048;
 constexpr int kNmSld = 68;  // padded row of 64 staged scales

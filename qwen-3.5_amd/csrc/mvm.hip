@@ -7,7 +7,7 @@
 // for each 8 rows and adds every column of every row with a 64-bit atomic; at 24 rows the MLP
 // spent 193 us on 38 MB of weights.  Here the products go to v_mfma_f32_16x16x32_bf16 and the
 // K splits leave plain f32 partials that a second kernel adds in split order.  Measured, 2B layer
-// calls: MLP at 24 rows 192.6 -> 33.6 us, DeltaNet at 9 rows 85.6 -> 27, the projections around the
+// calls: MLP at 24 rows 192.6 -> 31.8 us, DeltaNet at 9 rows 85.6 -> 27.8, the projections around the
 // attention of 16 rows 104 -> 24, q8_gemv 2048 x 6144 at 8 rows 35.0 -> 8.6.
 //
 // Arithmetic (f32 products): the int8 weight is exact in bf16; its block scale multiplies the input,
